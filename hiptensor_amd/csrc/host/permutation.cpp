@@ -37,7 +37,7 @@ namespace
     }
 
     // HIPTENSOR_AMD_PERMUTE="kernel[,tile[,maxvec[,group]]]": kernel is auto | gather | tiled |
-    // rows | strip | grouped (tiled and rows name the same preference: whichever of the two the
+    // rows | strip | grouped | runs (tiled and rows name the same preference: whichever of the two the
     // layout admits; strip and grouped - which includes the shared-fastest-mode tiles - are
     // taken wherever the layout admits them),
     // tile is 0..2 or -1, maxvec caps the vector width, group sets the band width of the
@@ -62,6 +62,8 @@ namespace
                 t.kernel = HIPTK_PERM_STRIP;
             else if(!std::strcmp(tok, "grouped"))
                 t.kernel = HIPTK_PERM_GROUPED;
+            else if(!std::strcmp(tok, "runs"))
+                t.kernel = HIPTK_PERM_RUNS;
             tok = strtok_r(nullptr, ",", &save);
         }
         if(tok)

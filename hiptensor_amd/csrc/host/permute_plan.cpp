@@ -313,8 +313,12 @@ namespace hipta
         int        kernel;
         if(tune.kernel == HIPTK_PERM_GROUPED && (tryGrouped(true, true) || tryShared(true)))
             return PermuteStatus::OK;
+        const int  full   = 16 / in.elem_bytes;
+        const bool runs   = shared && ext[0] >= full && cap >= full; // a 16-byte vector spans two runs at the most
         if(tune.kernel == HIPTK_PERM_GATHER)
             kernel = HIPTK_PERM_GATHER;
+        else if(tune.kernel == HIPTK_PERM_RUNS && runs)
+            kernel = HIPTK_PERM_RUNS;
         else if(tune.kernel == HIPTK_PERM_STRIP && (stripJ || stripI))
             kernel = HIPTK_PERM_STRIP;
         else if(tune.kernel == HIPTK_PERM_TILED || tune.kernel == HIPTK_PERM_ROWS)
@@ -334,6 +338,11 @@ namespace hipta
         out.kernel = kernel;
         if(kernel == HIPTK_PERM_GATHER)
             return PermuteStatus::OK;
+        if(kernel == HIPTK_PERM_RUNS)
+        {
+            out.vec_r = out.vec_w = full;
+            return PermuteStatus::OK;
+        }
 
         out.mode_i = 0;
         if(kernel == HIPTK_PERM_STRIP)
@@ -401,6 +410,31 @@ namespace hipta
             out.vec_r = out.vec_w = std::min(vr, vw);
             const int order[]     = {1, 0, 2};
             out.tile              = tune.tile >= 0 && tune.tile <= 2 ? tune.tile : pickTile(in.elem_bytes, ext[0], ext[mj], order);
+            // Vectors of the linear output instead of tiles, from 64-byte runs on (below, f16 24.500.700.8 ->
+            // (0,2,1,3): 122.6 us on these tiles, 95.4 linear, 65.0 on shared tiles), where
+            //   - the run is no multiple of 16 bytes: f32 21.79.79.20.8.7 -> (0,1,3,4,5,2) 443 -> 203 us, f16
+            //     229.60.25.24 -> (0,3,2,1) 22.3 -> 10.5, f16 33.500.700.8 -> (0,2,1,3) 430 -> 178;
+            //   - the tiles' lanes mostly fall outside: f32 30.7.61.7.7.65 -> (0,4,2,3,1,5) 468 -> 91 (11 % inside),
+            //     f16 40.64.128.256 -> (0,3,2,1) 116 -> 77 (31 %), f16 64.64.128.256 -> (0,2,1,3) 104 -> 96, f32
+            //     16.64.128.512 146 -> 130 (50 %; but f32 32.64.128.512, half of a square tile, 198 and 201);
+            //   - or a square tile cuts the run into 256 bytes, which only a tensor beyond the L2 minds: f32
+            //     128.64.128.200 -> (0,2,1,3) 301 -> 270, f16 256.64.128.256 378 -> 347.
+            // Whole runs of full vectors stay in tiles: f32 64.64.64.256 -> (0,3,2,1) 96 against 108,
+            // 256.64.128.128 341 and 347; and so do tensors of a launch's worth of latency (33.40.30 6.4 us on
+            // either, 64.40.30 6.3 and 6.5).
+            const Tile   tt     = (in.elem_bytes == 4 ? TILES4 : TILES2)[out.tile];
+            const double inside = coverage(ext[0], tt.ti) * coverage(ext[mj], tt.tj);
+            const bool   narrow = out.vec_r < full;
+            const bool   sparse = inside <= (in.elem_bytes == 4 && out.tile == 0 ? 0.45 : 0.55);
+            const bool   cut    = out.tile == 0 && ext[0] >= 2 * tt.ti && count >= (1 << 22);
+            if(runs && tune.kernel < 0 && tune.tile < 0 && count >= (1 << 17) && ext[0] * in.elem_bytes >= 64
+               && (narrow || sparse || cut))
+            {
+                out.kernel = HIPTK_PERM_RUNS;
+                out.mode_j = 0;
+                out.tile   = 0;
+                out.vec_r = out.vec_w = full;
+            }
         }
         return PermuteStatus::OK;
     }

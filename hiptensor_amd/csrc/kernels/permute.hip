@@ -18,6 +18,9 @@
 //             tile column B's two fastest modes, so that runs stay long when no single mode is.
 //   * SHARED  ROWS for a short shared fastest mode (interleaved channels): tiles of that mode
 //             times a chunk of A's next mode times a chunk of B's next mode, through LDS.
+//   * RUNS    ROWS without tiles: B is written front to back in 16-byte vectors, each thread finding
+//             where its vector's run lies in A; for runs that no tile covers well or whose odd
+//             length leaves ROWS only narrow vectors.
 //   * GATHER  one thread per element of B; covers tiny tensors and awkward extents.
 // Element operation per Composable Kernel's UnaryCombinedOp<Aop, Scale, Bop>
 // (ck/tensor_operation/gpu/element/combined_element_wise_operation.hpp:14-32): every step is
@@ -660,6 +663,124 @@ namespace hiptk
             static_cast<T*>(g.B)[idx] = element_op(static_cast<const T*>(g.A)[aoff], alpha, g.op_a, g.op_b);
         }
 
+        // 16 bytes at any multiple of the element
+        template <int ALIGN>
+        struct LooseBits;
+        template <>
+        struct LooseBits<2>
+        {
+            typedef uint32_t type __attribute__((ext_vector_type(4), aligned(2)));
+        };
+        template <>
+        struct LooseBits<4>
+        {
+            typedef uint32_t type __attribute__((ext_vector_type(4), aligned(4)));
+        };
+
+        struct RArgs
+        {
+            const void* A;
+            void*       B;
+            uint32_t    n; // elements
+            uint32_t    e0, m0; // extent of the shared fastest mode and its reciprocal
+            int32_t     nb; // the other modes, in B's order
+            uint32_t    ext[HIPTK_PERM_MAX_RANK - 1], astr[HIPTK_PERM_MAX_RANK - 1], magic[HIPTK_PERM_MAX_RANK - 1];
+            float       alpha;
+            int32_t     op_a, op_b;
+        };
+
+        // x / e and x % e by the reciprocal m = floor(2^32 / e) + 1, exact for every 32-bit x (the high word is the
+        // quotient or one more)
+        __device__ inline uint32_t div_by(uint32_t x, uint32_t e, uint32_t m, uint32_t& rem)
+        {
+            uint32_t q = __umulhi(x, m), r = x - q * e;
+            if((int32_t)r < 0)
+            {
+                q -= 1;
+                r += e;
+            }
+            rem = r;
+            return q;
+        }
+
+        // A and B share the fastest mode, of V = 16 bytes' worth of elements or more.  Bound by HBM.  A tile of two modes
+        // wastes the lanes that overhang them, and needs vectors that divide the run; here a vector is any V consecutive
+        // elements of B, taken from A in one load at whatever address they have there (global memory takes 16-byte loads
+        // and stores at any multiple of the element), or in two where the vector spans the end of a run.
+        // f32 21.79.79.20.8.7 -> (0,1,3,4,5,2), 587 MB: 443 us in tiles, 203 here (5.8 TB/s); f32 30.7.61.7.7.65 ->
+        // (0,4,2,3,1,5), 163 MB in runs of 120 bytes: 468 -> 91 us (3.6 TB/s: the run's ends share lines with others').
+        template <typename T>
+        __global__ __launch_bounds__(PERM_THREADS) void permute_runs_kernel(RArgs a)
+        {
+            constexpr int V = 16 / (int)sizeof(T);
+            constexpr int U = 4;
+            using raw_t     = typename LooseBits<sizeof(T)>::type;
+            struct Elems
+            {
+                T v[V];
+            };
+            const T* __restrict__ A = static_cast<const T*>(a.A);
+            T* __restrict__ B       = static_cast<T*>(a.B);
+            const T alpha           = static_cast<T>(a.alpha);
+            auto    load            = [&](uint32_t off) {
+                return __builtin_bit_cast(Elems, __builtin_nontemporal_load(reinterpret_cast<const raw_t*>(A + off)));
+            };
+
+            const uint32_t last  = a.n - V; // the last vector is moved back to end with the tensor
+            const uint32_t first = (blockIdx.x * (PERM_THREADS * U) + threadIdx.x) * V;
+            uint32_t       src[U], next[U], left[U]; // the vector's place in A, that of its next run, elements of this run from it on
+            Elems          x[U];
+#pragma unroll
+            for(int u = 0; u < U; ++u)
+            {
+                const uint32_t at  = first + u * PERM_THREADS * V;
+                const uint32_t idx = at < last ? at : last;
+                uint32_t       pos, off = 0, noff = 0;
+                uint32_t       rem   = div_by(idx, a.e0, a.m0, pos);
+                bool           carry = true; // the next run's coordinates: one more, from the fastest mode up
+                for(int d = 0; d < a.nb; ++d)
+                {
+                    uint32_t c;
+                    rem = div_by(rem, a.ext[d], a.magic[d], c);
+                    const uint32_t c1 = !carry ? c : c + 1 == a.ext[d] ? 0u : c + 1;
+                    off += c * a.astr[d];
+                    noff += c1 * a.astr[d];
+                    carry = carry && c1 == 0;
+                }
+                src[u]  = off + pos;
+                next[u] = noff;
+                left[u] = a.e0 - pos;
+                x[u]    = load(src[u] < last ? src[u] : last);
+            }
+#pragma unroll
+            for(int u = 0; u < U; ++u)
+            {
+                if(left[u] < V)
+                {
+                    const uint32_t k = left[u];
+                    if(src[u] <= last && next[u] >= k)
+                    {
+                        const Elems y = load(next[u] - k);
+#pragma unroll
+                        for(int e = 1; e < V; ++e)
+                            x[u].v[e] = (uint32_t)e < k ? x[u].v[e] : y.v[e];
+                    }
+                    else // one of the two vectors would reach beyond the ends of A
+                    {
+#pragma unroll
+                        for(int e = 0; e < V; ++e)
+                            x[u].v[e] = A[(uint32_t)e < k ? src[u] + e : next[u] + (e - k)];
+                    }
+                }
+                const uint32_t at = first + u * PERM_THREADS * V;
+#pragma unroll
+                for(int e = 0; e < V; ++e)
+                    x[u].v[e] = element_op(x[u].v[e], alpha, a.op_a, a.op_b);
+                if(at < a.n)
+                    __builtin_nontemporal_store(__builtin_bit_cast(raw_t, x[u]), reinterpret_cast<raw_t*>(B + (at < last ? at : last)));
+            }
+        }
+
         // ---------------------------------------------------------------- host side
 
         struct TileShape
@@ -930,6 +1051,10 @@ extern "C" const char* hiptk_permute_kernel_name(const hiptk_permute_t* p)
         break;
     }
     case HIPTK_PERM_GATHER: snprintf(name, sizeof(name), "permute_gather_%s", type_tag(p->elem_bytes)); break;
+    case HIPTK_PERM_RUNS:
+        if(p->vec_r * p->elem_bytes == 16 && p->vec_w == p->vec_r)
+            snprintf(name, sizeof(name), "permute_runs_%s_%d_v%d", type_tag(p->elem_bytes), p->extent[0], p->vec_r);
+        break;
     case HIPTK_PERM_GROUPED:
         if(vec_allowed(p->elem_bytes, p->vec_r) && vec_allowed(p->elem_bytes, p->vec_w) && p->chunk_i >= 1 && p->chunk_j >= 1)
             snprintf(name,
@@ -1026,6 +1151,49 @@ extern "C" int hiptk_permute(const hiptk_permute_t* p, const void* A, void* B, v
             hipLaunchKernelGGL((permute_gather_kernel<float>), dim3(grid), dim3(PERM_THREADS), 0, s, g);
         else
             hipLaunchKernelGGL((permute_gather_kernel<_Float16>), dim3(grid), dim3(PERM_THREADS), 0, s, g);
+        rc = (int)hipGetLastError();
+    }
+    else if(p->kernel == HIPTK_PERM_RUNS)
+    {
+        const int v = 16 / p->elem_bytes;
+        if(p->vec_r != v || p->vec_w != v)
+            return HIPTK_ERR_NO_KERNEL;
+        // one run at least in every vector's reach, so that a vector spans two at the most; the reciprocals want
+        // divisors of 2 and more
+        if(p->rank < 2 || p->b_stride[0] != 1 || p->extent[0] < v)
+            return HIPTK_ERR_ARG;
+        RArgs a;
+        memset(&a, 0, sizeof(a));
+        a.A     = A;
+        a.B     = B;
+        a.n     = (uint32_t)n;
+        a.e0    = (uint32_t)p->extent[0];
+        a.m0    = magic_of(a.e0);
+        a.alpha = p->alpha;
+        a.op_a  = p->op_a;
+        a.op_b  = p->op_b;
+        int order[HIPTK_PERM_MAX_RANK];
+        for(int d = 0; d < p->rank; ++d)
+            order[d] = d;
+        std::sort(order + 1, order + p->rank, [p](int x, int y) {
+            return p->b_stride[x] != p->b_stride[y] ? p->b_stride[x] < p->b_stride[y] : x < y;
+        });
+        for(int k = 1; k < p->rank; ++k)
+        {
+            const int d = order[k];
+            if(p->extent[d] == 1)
+                continue;
+            a.ext[a.nb]   = (uint32_t)p->extent[d];
+            a.astr[a.nb]  = (uint32_t)p->a_stride[d];
+            a.magic[a.nb] = magic_of((uint32_t)p->extent[d]);
+            ++a.nb;
+        }
+        const int64_t  per  = (int64_t)PERM_THREADS * 4 * v;
+        const uint32_t grid = (uint32_t)((n + per - 1) / per);
+        if(p->elem_bytes == 4)
+            hipLaunchKernelGGL((permute_runs_kernel<float>), dim3(grid), dim3(PERM_THREADS), 0, s, a);
+        else
+            hipLaunchKernelGGL((permute_runs_kernel<_Float16>), dim3(grid), dim3(PERM_THREADS), 0, s, a);
         rc = (int)hipGetLastError();
     }
     else if(p->kernel == HIPTK_PERM_TILED || p->kernel == HIPTK_PERM_ROWS)

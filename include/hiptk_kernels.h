@@ -205,11 +205,14 @@ enum
                               column width_j elements of mode_j and, when width_j == extent[mode_j],
                               chunk_j indices of B's next mode (mode_j2, contiguous in B); a second
                               mode may be absent (-1, chunk 1)                                    */
-    HIPTK_PERM_SHARED = 6  /* ROWS for a short shared fastest mode (at most 128 elements, e.g. the
+    HIPTK_PERM_SHARED = 6, /* ROWS for a short shared fastest mode (at most 128 elements, e.g. the
                               four channels of RGBA pixels): a tile is mode 0 times chunk_i indices of
                               A's next mode (mode_i2) times chunk_j indices of B's next mode (mode_j2);
                               it is read in runs of extent[0] * chunk_i and, through LDS, written in
                               runs of extent[0] * chunk_j                                        */
+    HIPTK_PERM_RUNS = 7    /* ROWS without tiles: B is written front to back in 16-byte vectors taken
+                              from A at any element address; mode 0 is shared and holds at least one
+                              vector (vec_r == vec_w == 16 / elem_bytes, no alignment asked for)   */
 };
 
 #define HIPTK_PERM_MAX_RANK 6
