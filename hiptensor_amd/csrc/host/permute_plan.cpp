@@ -268,6 +268,14 @@ namespace hipta
             out.width_j = (int32_t)wj;
             out.vec_r   = vr;
             out.vec_w   = vw;
+            // Where an odd extent would leave narrow vectors: 16-byte ones at any element, if both sides of the tile are
+            // 64 elements or more (f16 126 x 125 43.4 -> 29.4 us, 128 x 65 14.2 -> 8.4, f32 105 x 125 53.6 -> 43.0; but f16
+            // 120 x 51 257 -> 278: the vector moved back at a short run's end weighs more).
+            if(const int full = 16 / in.elem_bytes; cap >= full && std::min(vr, vw) < full && wi * ci >= 64 && wj * cj >= 64)
+            {
+                out.loose = 1;
+                out.vec_r = out.vec_w = full;
+            }
             return true;
         };
         // A short shared fastest mode (interleaved channels): tiles of that mode times a chunk of

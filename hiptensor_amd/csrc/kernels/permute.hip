@@ -32,6 +32,7 @@
 #include <algorithm>
 #include <cstdio>
 #include <cstring>
+#include <type_traits>
 
 #include "hiptk_kernels.h"
 
@@ -114,6 +115,34 @@ namespace hiptk
         __device__ inline void store_stream(T* p, const Vec<T, V>& v)
         {
             using R = typename RawBits<sizeof(T) * V>::type;
+            __builtin_nontemporal_store(__builtin_bit_cast(R, v), reinterpret_cast<R*>(p));
+        }
+
+        // 16 bytes at any multiple of the element
+        template <int ALIGN>
+        struct LooseBits;
+        template <>
+        struct LooseBits<2>
+        {
+            typedef uint32_t type __attribute__((ext_vector_type(4), aligned(2)));
+        };
+        template <>
+        struct LooseBits<4>
+        {
+            typedef uint32_t type __attribute__((ext_vector_type(4), aligned(4)));
+        };
+
+        template <typename T>
+        __device__ inline Vec<T, 16 / (int)sizeof(T)> load_loose(const T* p)
+        {
+            using R = typename LooseBits<sizeof(T)>::type;
+            return __builtin_bit_cast(Vec<T, 16 / (int)sizeof(T)>, __builtin_nontemporal_load(reinterpret_cast<const R*>(p)));
+        }
+
+        template <typename T>
+        __device__ inline void store_loose(T* p, const Vec<T, 16 / (int)sizeof(T)>& v)
+        {
+            using R = typename LooseBits<sizeof(T)>::type;
             __builtin_nontemporal_store(__builtin_bit_cast(R, v), reinterpret_cast<R*>(p));
         }
 
@@ -406,6 +435,12 @@ namespace hiptk
             }
         }
 
+        // 2^32 / d rounded up, d >= 2: __umulhi(v, recip(d)) == v / d while v * d < 2^32
+        __device__ inline uint32_t recip(uint32_t d)
+        {
+            return 0xFFFFFFFFu / d + 1u;
+        }
+
         struct QArgs
         {
             const void* A;
@@ -428,7 +463,13 @@ namespace hiptk
         // contiguous in A, so a row is one run of A.  Column y is (y0, y1) over mode j and B's next
         // mode in the same way, one run of B.  Rows are read along x, the tile is parked in LDS as
         // [y][x], and columns are written along y.
-        template <typename T, int VR, int VW>
+        // Narrow vectors are bound by the number of accesses, not by their bytes.  LOOSE: 16-byte vectors
+        // whatever the extents; they start at any element, and the last one of a run is moved back to end with it
+        // (its first elements are moved twice, to the same place).  Runs shorter than a vector, which only the
+        // ragged tiles at the edges have, are moved by elements.
+        // f16 21.25.23.57.25 -> (4,2,1,3,0), 34 MB: 43.4 -> 29.4 us; f16 129.513.65 -> (2,0,1) 14.2 -> 8.4; f32 21.25.23.57.25
+        // 53.6 -> 43.0; f32 28.24.12.47.19.37 -> (4,2,3,0,5,1), 1 GB: 684 -> 634.
+        template <typename T, int VR, int VW, bool LOOSE>
         __global__ __launch_bounds__(PERM_THREADS) void permute_group_kernel(QArgs a)
         {
             constexpr int NT = PERM_THREADS;
@@ -465,53 +506,83 @@ namespace hiptk
             const uint32_t cj = (a.e_j1 - j1s) < a.c_j ? (a.e_j1 - j1s) : a.c_j;
             // rows and columns inside the extents (c > 1 only with the whole first mode: w == e)
             const uint32_t nx = a.w_i * (ci - 1) + wi, ny = a.w_j * (cj - 1) + wj;
-            const uint32_t RV = a.w_i * a.c_i / VR, CV = a.w_j * a.c_j / VW; // vectors per nominal row / column
+            // vectors per nominal row / column
+            const uint32_t RV = (a.w_i * a.c_i + (LOOSE ? VR - 1 : 0)) / VR, CV = (a.w_j * a.c_j + (LOOSE ? VW - 1 : 0)) / VW;
             aoff += i0s + i1s * a.e_i0 + j0s * a.a_j0 + j1s * a.a_j1;
             boff += i0s * a.b_i0 + i1s * a.b_i1 + j0s + j1s * a.e_j0;
             const T alpha = static_cast<T>(a.alpha);
 
-            const uint32_t total_r = RV * ny;
-            for(uint32_t u0 = 0; u0 < total_r; u0 += NT * U)
-            {
-                Vec<T, VR> r[U];
-                uint32_t   at[U];
-#pragma unroll
-                for(int k = 0; k < U; ++k)
+            auto read = [&](auto width, uint32_t per_row, uint32_t m_row) {
+                constexpr int  W     = decltype(width)::value;
+                const uint32_t total = per_row * ny;
+                for(uint32_t u0 = 0; u0 < total; u0 += NT * U)
                 {
-                    const uint32_t v  = u0 + tid + k * NT;
-                    const uint32_t y  = __umulhi(v, a.m_rv), xv = v - y * RV;
-                    const uint32_t y1 = __umulhi(y, a.m_wj), y0 = y - y1 * a.w_j;
-                    const bool     ok = v < total_r && xv * VR < nx;
-                    at[k]             = ok ? y * a.pitch + xv * VR : 0xFFFFFFFFu;
-                    // out-of-range lanes load the tile's first element: no branch, all loads in flight
-                    r[k] = load_stream<T, VR>(A + aoff + (ok ? xv * VR + y0 * a.a_j0 + y1 * a.a_j1 : 0u));
-                }
+                    Vec<T, W> r[U];
+                    uint32_t  at[U];
 #pragma unroll
-                for(int k = 0; k < U; ++k)
-                {
-                    if(at[k] != 0xFFFFFFFFu)
+                    for(int k = 0; k < U; ++k)
                     {
+                        const uint32_t v  = u0 + tid + k * NT;
+                        const uint32_t y  = __umulhi(v, m_row);
+                        uint32_t       x  = (v - y * per_row) * W;
+                        const uint32_t y1 = __umulhi(y, a.m_wj), y0 = y - y1 * a.w_j;
+                        const bool     ok = v < total && x < nx;
+                        if constexpr(LOOSE)
+                            x = x + W > nx ? nx - W : x;
+                        at[k] = ok ? y * a.pitch + x : 0xFFFFFFFFu;
+                        // out-of-range lanes load the tile's first element: no branch, all loads in flight
+                        const T* from = A + aoff + (ok ? x + y0 * a.a_j0 + y1 * a.a_j1 : 0u);
+                        if constexpr(LOOSE && W > 1)
+                            r[k] = load_loose(from);
+                        else
+                            r[k] = load_stream<T, W>(from);
+                    }
 #pragma unroll
-                        for(int e = 0; e < VR; ++e)
-                            tile[at[k] + e] = element_op(r[k].v[e], alpha, a.op_a, a.op_b);
+                    for(int k = 0; k < U; ++k)
+                    {
+                        if(at[k] != 0xFFFFFFFFu)
+                        {
+#pragma unroll
+                            for(int e = 0; e < W; ++e)
+                                tile[at[k] + e] = element_op(r[k].v[e], alpha, a.op_a, a.op_b);
+                        }
                     }
                 }
-            }
-            __syncthreads();
-            const uint32_t total_w = CV * nx;
-            for(uint32_t v = tid; v < total_w; v += NT)
-            {
-                const uint32_t x = __umulhi(v, a.m_cv), yv = v - x * CV;
-                if(yv * VW < ny)
+            };
+            auto write = [&](auto width, uint32_t per_col, uint32_t m_col) {
+                constexpr int  W     = decltype(width)::value;
+                const uint32_t total = per_col * nx;
+                for(uint32_t v = tid; v < total; v += NT)
                 {
-                    const uint32_t x1 = __umulhi(x, a.m_wi), x0 = x - x1 * a.w_i;
-                    Vec<T, VW>     o;
+                    const uint32_t x = __umulhi(v, m_col);
+                    uint32_t       y = (v - x * per_col) * W;
+                    if(y < ny)
+                    {
+                        if constexpr(LOOSE)
+                            y = y + W > ny ? ny - W : y;
+                        const uint32_t x1 = __umulhi(x, a.m_wi), x0 = x - x1 * a.w_i;
+                        Vec<T, W>      o;
 #pragma unroll
-                    for(int e = 0; e < VW; ++e)
-                        o.v[e] = tile[(yv * VW + e) * a.pitch + x];
-                    store_stream<T, VW>(B + boff + yv * VW + x0 * a.b_i0 + x1 * a.b_i1, o);
+                        for(int e = 0; e < W; ++e)
+                            o.v[e] = tile[(y + e) * a.pitch + x];
+                        T* to = B + boff + y + x0 * a.b_i0 + x1 * a.b_i1;
+                        if constexpr(LOOSE && W > 1)
+                            store_loose(to, o);
+                        else
+                            store_stream<T, W>(to, o);
+                    }
                 }
-            }
+            };
+            typedef std::integral_constant<int, 1> One;
+            if(!LOOSE || nx >= VR)
+                read(std::integral_constant<int, VR>{}, RV, a.m_rv);
+            else
+                read(One{}, nx < 2 ? 2 : nx, recip(nx < 2 ? 2 : nx));
+            __syncthreads();
+            if(!LOOSE || ny >= VW)
+                write(std::integral_constant<int, VW>{}, CV, a.m_cv);
+            else
+                write(One{}, ny < 2 ? 2 : ny, recip(ny < 2 ? 2 : ny));
         }
 
         struct HArgs
@@ -663,20 +734,6 @@ namespace hiptk
             static_cast<T*>(g.B)[idx] = element_op(static_cast<const T*>(g.A)[aoff], alpha, g.op_a, g.op_b);
         }
 
-        // 16 bytes at any multiple of the element
-        template <int ALIGN>
-        struct LooseBits;
-        template <>
-        struct LooseBits<2>
-        {
-            typedef uint32_t type __attribute__((ext_vector_type(4), aligned(2)));
-        };
-        template <>
-        struct LooseBits<4>
-        {
-            typedef uint32_t type __attribute__((ext_vector_type(4), aligned(4)));
-        };
-
         struct RArgs
         {
             const void* A;
@@ -714,17 +771,11 @@ namespace hiptk
         {
             constexpr int V = 16 / (int)sizeof(T);
             constexpr int U = 4;
-            using raw_t     = typename LooseBits<sizeof(T)>::type;
-            struct Elems
-            {
-                T v[V];
-            };
+            typedef Vec<T, V> Elems;
             const T* __restrict__ A = static_cast<const T*>(a.A);
             T* __restrict__ B       = static_cast<T*>(a.B);
             const T alpha           = static_cast<T>(a.alpha);
-            auto    load            = [&](uint32_t off) {
-                return __builtin_bit_cast(Elems, __builtin_nontemporal_load(reinterpret_cast<const raw_t*>(A + off)));
-            };
+            auto    load            = [&](uint32_t off) { return load_loose(A + off); };
 
             const uint32_t last  = a.n - V; // the last vector is moved back to end with the tensor
             const uint32_t first = (blockIdx.x * (PERM_THREADS * U) + threadIdx.x) * V;
@@ -777,7 +828,7 @@ namespace hiptk
                 for(int e = 0; e < V; ++e)
                     x[u].v[e] = element_op(x[u].v[e], alpha, a.op_a, a.op_b);
                 if(at < a.n)
-                    __builtin_nontemporal_store(__builtin_bit_cast(raw_t, x[u]), reinterpret_cast<raw_t*>(B + (at < last ? at : last)));
+                    store_loose(B + (at < last ? at : last), x[u]);
             }
         }
 
@@ -917,12 +968,17 @@ namespace hiptk
         }
 
         template <typename T, int VMAX>
-        int launch_group(int vr, int vw, const QArgs& a, uint32_t grid, size_t lds, hipStream_t s)
+        int launch_group(int vr, int vw, bool loose, const QArgs& a, uint32_t grid, size_t lds, hipStream_t s)
         {
+            if(loose)
+            {
+                hipLaunchKernelGGL((permute_group_kernel<T, VMAX, VMAX, true>), dim3(grid), dim3(PERM_THREADS), lds, s, a);
+                return (int)hipGetLastError();
+            }
 #define HIPTK_GROUP_CASE(R, W)                                                                                     \
     if(vr == R && vw == W)                                                                                         \
     {                                                                                                              \
-        hipLaunchKernelGGL((permute_group_kernel<T, R, W>), dim3(grid), dim3(PERM_THREADS), lds, s, a);              \
+        hipLaunchKernelGGL((permute_group_kernel<T, R, W, false>), dim3(grid), dim3(PERM_THREADS), lds, s, a);              \
         return (int)hipGetLastError();                                                                             \
     }
             HIPTK_GROUP_CASE(1, 1)
@@ -1059,7 +1115,7 @@ extern "C" const char* hiptk_permute_kernel_name(const hiptk_permute_t* p)
         if(vec_allowed(p->elem_bytes, p->vec_r) && vec_allowed(p->elem_bytes, p->vec_w) && p->chunk_i >= 1 && p->chunk_j >= 1)
             snprintf(name,
                      sizeof(name),
-                     "permute_grouped_%s_%dx%d_r%d_w%d",
+                     p->loose ? "permute_grouped_%s_%dx%d_r%d_w%d_loose" : "permute_grouped_%s_%dx%d_r%d_w%d",
                      type_tag(p->elem_bytes),
                      p->width_i * p->chunk_i,
                      p->width_j * p->chunk_j,
@@ -1279,16 +1335,23 @@ extern "C" int hiptk_permute(const hiptk_permute_t* p, const void* A, void* B, v
             return HIPTK_ERR_ARG;
         // vectors: whole vectors inside the tile widths and the fastest modes, every other stride
         // and both bases aligned
-        const int vr = p->vec_r, vw = p->vec_w;
-        if(p->extent[0] % vr != 0 || p->extent[mj] % vw != 0 || w_i % vr != 0 || w_j % vw != 0 || !aligned(A, vr * p->elem_bytes)
-           || !aligned(B, vw * p->elem_bytes))
+        // (loose: 16 bytes at any element)
+        const int  vr = p->vec_r, vw = p->vec_w;
+        const bool loose = p->loose != 0;
+        if(loose && (vr * p->elem_bytes != 16 || vw != vr))
             return HIPTK_ERR_ARG;
-        for(int d = 1; d < p->rank; ++d)
-            if(p->a_stride[d] % vr != 0)
+        if(!loose)
+        {
+            if(p->extent[0] % vr != 0 || p->extent[mj] % vw != 0 || w_i % vr != 0 || w_j % vw != 0
+               || !aligned(A, vr * p->elem_bytes) || !aligned(B, vw * p->elem_bytes))
                 return HIPTK_ERR_ARG;
-        for(int d = 0; d < p->rank; ++d)
-            if(d != mj && p->b_stride[d] % vw != 0)
-                return HIPTK_ERR_ARG;
+            for(int d = 1; d < p->rank; ++d)
+                if(p->a_stride[d] % vr != 0)
+                    return HIPTK_ERR_ARG;
+            for(int d = 0; d < p->rank; ++d)
+                if(d != mj && p->b_stride[d] % vw != 0)
+                    return HIPTK_ERR_ARG;
+        }
 
         QArgs a;
         memset(&a, 0, sizeof(a));
@@ -1318,9 +1381,9 @@ extern "C" int hiptk_permute(const hiptk_permute_t* p, const void* A, void* B, v
         const size_t lds = (size_t)TJ * a.pitch * p->elem_bytes;
         if(lds > (size_t)GROUP_MAX_LDS || TI / vr < 2 || TJ / vw < 2 || w_i < 2 || w_j < 2)
             return HIPTK_ERR_ARG; // (the reciprocals below are exact for divisors of 2 and more)
-        a.m_rv = magic_of(TI / vr);
+        a.m_rv = magic_of(loose ? (TI + vr - 1) / vr : TI / vr);
         a.m_wj = magic_of(a.w_j);
-        a.m_cv = magic_of(TJ / vw);
+        a.m_cv = magic_of(loose ? (TJ + vw - 1) / vw : TJ / vw);
         a.m_wi = magic_of(a.w_i);
         a.alpha = p->alpha;
         a.op_a  = p->op_a;
@@ -1338,8 +1401,8 @@ extern "C" int hiptk_permute(const hiptk_permute_t* p, const void* A, void* B, v
         }
         if(grid >= (int64_t(1) << 31))
             return HIPTK_ERR_ARG;
-        rc = p->elem_bytes == 4 ? launch_group<float, 4>(vr, vw, a, (uint32_t)grid, lds, s)
-                                : launch_group<_Float16, 8>(vr, vw, a, (uint32_t)grid, lds, s);
+        rc = p->elem_bytes == 4 ? launch_group<float, 4>(vr, vw, loose, a, (uint32_t)grid, lds, s)
+                                : launch_group<_Float16, 8>(vr, vw, loose, a, (uint32_t)grid, lds, s);
     }
     else if(p->kernel == HIPTK_PERM_SHARED)
     {

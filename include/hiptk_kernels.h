@@ -240,6 +240,8 @@ typedef struct hiptk_permute
     int32_t mode_i2, mode_j2; /* GROUPED: the second row / column mode, or -1                     */
     int32_t chunk_i, chunk_j; /* GROUPED: indices of mode_i2 / mode_j2 per tile (1 when absent)   */
     int32_t width_i, width_j; /* GROUPED: elements of mode 0 / mode_j per tile                    */
+    int32_t loose; /* GROUPED: 16-byte vectors that start at any element and need divide nothing
+                      (vec_r == vec_w == 16 / elem_bytes)                                         */
 } hiptk_permute_t;
 
 /* Name of the kernel a problem selects ("" if the combination is not instantiated). */
