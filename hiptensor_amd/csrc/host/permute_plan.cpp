@@ -268,10 +268,18 @@ namespace hipta
             out.width_j = (int32_t)wj;
             out.vec_r   = vr;
             out.vec_w   = vw;
-            // Where an odd extent would leave narrow vectors: 16-byte ones at any element, if both sides of the tile are
+            // Where the extents would leave narrow vectors: 16-byte ones at any element, if both sides of the tile are
             // 64 elements or more (f16 126 x 125 43.4 -> 29.4 us, 128 x 65 14.2 -> 8.4, f32 105 x 125 53.6 -> 43.0; but f16
-            // 120 x 51 257 -> 278: the vector moved back at a short run's end weighs more).
-            if(const int full = 16 / in.elem_bytes; cap >= full && std::min(vr, vw) < full && wi * ci >= 64 && wj * cj >= 64)
+            // 120 x 51 257 -> 278: the vector moved back at a short run's end weighs more).  Pairs of f16 are 4-byte
+            // accesses already: they lose to it only while the tensor fits the L2 and the accesses are what counts (up
+            // to 2^23 elements 0.70-0.98 of the pairs' time; beyond, 188 random shapes 0.68-1.57, half of them slower:
+            // 138.16.70.18.82 -> (2,1,4,0,3) 388 us in pairs, 537 loose).  A side of single elements is worth it at any
+            // size (0.51-1.0), next to pairs on the other side from columns of 120 elements on (0.55-0.99; shorter
+            // ones 0.72-1.20).  f32 gains over the whole range (0.73-1.04).
+            const int  full   = 16 / in.elem_bytes;
+            const int  narrow = std::min(vr, vw), wide = std::max(vr, vw);
+            const bool gains  = in.elem_bytes == 4 || count <= (1 << 23) || (narrow == 1 && (wide != 2 || wj * cj >= 120));
+            if(cap >= full && narrow < full && wi * ci >= 64 && wj * cj >= 64 && gains)
             {
                 out.loose = 1;
                 out.vec_r = out.vec_w = full;

@@ -132,6 +132,23 @@ def test_vector_width_follows_pointer_alignment(host_handle):
     assert _info(h, "f16", [64, 64, 64], [0, 1, 2], A=0x1008, B=0x2000)["vec_r"] == 4
 
 
+@pytest.mark.parametrize("dtype,lens,perm,name", [
+    # pairs of f16 on large tensors: the extents' own vectors (16-byte ones at any element are up to 1.5x slower there)
+    ("f16", [138, 16, 70, 18, 82], [2, 1, 4, 0, 3], "permute_grouped_f16_128x70_r2_w2"),
+    ("f16", [72, 52, 312, 36], [3, 2, 0, 1], "permute_grouped_f16_128x108_r8_w2"),
+    ("f16", [100, 16, 12, 48, 16, 8], [3, 5, 2, 0, 4, 1], "permute_grouped_f16_100x96_r2_w8"),
+    ("f16", [638, 52, 95, 51], [3, 2, 1, 0], "permute_grouped_f16_128x102_r2_w1"),
+    # ... smaller tensors, single elements and f32: 16-byte vectors at any element
+    ("f16", [154, 68, 562], [1, 0, 2], "permute_grouped_f16_128x68_r8_w8_loose"),
+    ("f16", [21, 25, 23, 57, 25], [4, 2, 1, 3, 0], "permute_grouped_f16_126x125_r8_w8_loose"),
+    ("f16", [7, 32, 32, 32, 16, 8], [5, 4, 1, 3, 2, 0], "permute_grouped_f16_126x128_r8_w8_loose"),
+    ("f16", [19, 11, 13, 33, 12, 23], [4, 2, 0, 3, 5, 1], "permute_grouped_f16_114x120_r8_w8_loose"),
+    ("f32", [154, 252, 240, 26], [3, 1, 2, 0], "permute_grouped_f32_128x104_r4_w4_loose"),
+])
+def test_vectors_at_any_element_where_they_gain(host_handle, dtype, lens, perm, name):
+    assert _info(host_handle, dtype, lens, perm)["kernel_name"] == name
+
+
 def test_every_validation_case_plans(host_handle):
     for rank in (2, 3, 4, 5, 6):
         for w in perm_cases.validation(rank, thin=36):
