@@ -766,11 +766,11 @@ namespace hiptk
         // and stores at any multiple of the element), or in two where the vector spans the end of a run.
         // f32 21.79.79.20.8.7 -> (0,1,3,4,5,2), 587 MB: 443 us in tiles, 203 here (5.8 TB/s); f32 30.7.61.7.7.65 ->
         // (0,4,2,3,1,5), 163 MB in runs of 120 bytes: 468 -> 91 us (3.6 TB/s: the run's ends share lines with others').
-        template <typename T>
+        // A thread moves U vectors, its loads all in flight.
+        template <typename T, int U>
         __global__ __launch_bounds__(PERM_THREADS) void permute_runs_kernel(RArgs a)
         {
             constexpr int V = 16 / (int)sizeof(T);
-            constexpr int U = 4;
             typedef Vec<T, V> Elems;
             const T* __restrict__ A = static_cast<const T*>(a.A);
             T* __restrict__ B       = static_cast<T*>(a.B);
@@ -833,6 +833,16 @@ namespace hiptk
         }
 
         // ---------------------------------------------------------------- host side
+
+        // Vectors per thread of the RUNS kernel.  Four keep more loads in flight, but a tensor of a few MB then makes too few
+        // workgroups for 256 compute units and the kernel lasts as long as one thread (2^17 f32: 32 workgroups): f32
+        // 16.20.4.8.8.4 -> (0,1,4,3,5,2) 5.7 us, 3.9 in tiles; one per thread takes 0.58-0.75 of four's time up to 2^20
+        // f32 (0.60-0.72 up to 2^21 f16), 0.87-0.91 just below the line here and 0.94-1.02 beyond it, with cases of up
+        // to 1.24.  From four workgroups of four a compute unit on, four.
+        int runs_per_thread(int64_t n, int v)
+        {
+            return n >= (int64_t(1) << 20) * v ? 4 : 1;
+        }
 
         struct TileShape
         {
@@ -1109,7 +1119,7 @@ extern "C" const char* hiptk_permute_kernel_name(const hiptk_permute_t* p)
     case HIPTK_PERM_GATHER: snprintf(name, sizeof(name), "permute_gather_%s", type_tag(p->elem_bytes)); break;
     case HIPTK_PERM_RUNS:
         if(p->vec_r * p->elem_bytes == 16 && p->vec_w == p->vec_r)
-            snprintf(name, sizeof(name), "permute_runs_%s_%d_v%d", type_tag(p->elem_bytes), p->extent[0], p->vec_r);
+            snprintf(name, sizeof(name), "permute_runs_%s_%d_v%dx%d", type_tag(p->elem_bytes), p->extent[0], p->vec_r, runs_per_thread(n, p->vec_r));
         break;
     case HIPTK_PERM_GROUPED:
         if(vec_allowed(p->elem_bytes, p->vec_r) && vec_allowed(p->elem_bytes, p->vec_w) && p->chunk_i >= 1 && p->chunk_j >= 1)
@@ -1244,12 +1254,17 @@ extern "C" int hiptk_permute(const hiptk_permute_t* p, const void* A, void* B, v
             a.magic[a.nb] = magic_of((uint32_t)p->extent[d]);
             ++a.nb;
         }
-        const int64_t  per  = (int64_t)PERM_THREADS * 4 * v;
+        const int      u    = runs_per_thread(n, v);
+        const int64_t  per  = (int64_t)PERM_THREADS * u * v;
         const uint32_t grid = (uint32_t)((n + per - 1) / per);
-        if(p->elem_bytes == 4)
-            hipLaunchKernelGGL((permute_runs_kernel<float>), dim3(grid), dim3(PERM_THREADS), 0, s, a);
+        if(p->elem_bytes == 4 && u == 4)
+            hipLaunchKernelGGL((permute_runs_kernel<float, 4>), dim3(grid), dim3(PERM_THREADS), 0, s, a);
+        else if(p->elem_bytes == 4)
+            hipLaunchKernelGGL((permute_runs_kernel<float, 1>), dim3(grid), dim3(PERM_THREADS), 0, s, a);
+        else if(u == 4)
+            hipLaunchKernelGGL((permute_runs_kernel<_Float16, 4>), dim3(grid), dim3(PERM_THREADS), 0, s, a);
         else
-            hipLaunchKernelGGL((permute_runs_kernel<_Float16>), dim3(grid), dim3(PERM_THREADS), 0, s, a);
+            hipLaunchKernelGGL((permute_runs_kernel<_Float16, 1>), dim3(grid), dim3(PERM_THREADS), 0, s, a);
         rc = (int)hipGetLastError();
     }
     else if(p->kernel == HIPTK_PERM_TILED || p->kernel == HIPTK_PERM_ROWS)

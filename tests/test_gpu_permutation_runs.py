@@ -33,6 +33,19 @@ def test_runs(gpu_handle, oracle_mod, dtype, shift):
     assert used == sum(lens[0] * wl.ELEM_BYTES[dtype] >= 16 for lens, _ in SHAPES)
 
 
+@pytest.mark.parametrize("dtype,lens", [("f32", [63, 256, 261]), ("f16", [127, 256, 259])])
+@pytest.mark.parametrize("shift", [(0, 0), (1, 3)])
+def test_four_vectors_a_thread(gpu_handle, oracle_mod, dtype, lens, shift):
+    """Just over the line from which a thread moves four vectors; the last workgroup holds few."""
+    w = wl.permutation(dtype, lens, [0, 2, 1], 1.7, dtype, *perm_cases.OPS[0])
+    A = wl.permutation_input(w)
+    print(f"[case] {dtype} {lens} shift {shift}", flush=True)
+    with _Override("runs"):
+        got, info = gpu_util.run_gpu_permutation(gpu_handle, w, A, a_shift=shift[0], b_shift=shift[1], return_info=True)
+    assert info["kernel_name"].endswith("x4"), info["kernel_name"]
+    assert _same(got, oracle_mod.permute(w, A))
+
+
 @pytest.mark.parametrize("dtype,lens,perm", [("f32", [30, 7, 61, 7, 7, 13], [0, 4, 2, 3, 1, 5]), ("f16", [229, 60, 25, 4], [0, 3, 2, 1]),
                                              ("f32", [128, 32, 48, 24], [0, 2, 1, 3])])
 def test_default_choice(gpu_handle, oracle_mod, dtype, lens, perm):

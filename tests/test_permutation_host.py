@@ -2,6 +2,7 @@
 reference's order (library/src/permutation/hiptensor_permutation.cpp:77-155, 173-189), mode
 fusion and kernel choice of the planner."""
 import ctypes as C
+import os
 
 import pytest
 
@@ -147,6 +148,34 @@ def test_vector_width_follows_pointer_alignment(host_handle):
 ])
 def test_vectors_at_any_element_where_they_gain(host_handle, dtype, lens, perm, name):
     assert _info(host_handle, dtype, lens, perm)["kernel_name"] == name
+
+
+@pytest.mark.parametrize("dtype,lens,perm,name", [
+    # a few MB: one vector per thread, so that there are workgroups enough (32.8.16.40: 160 and not 40)
+    ("f32", [32, 8, 16, 40], [0, 3, 2, 1], "permute_runs_f32_32_v4x1"),
+    ("f32", [55, 50, 16, 9], [0, 2, 1, 3], "permute_runs_f32_55_v4x1"),
+    ("f16", [41, 326, 156], [0, 2, 1], "permute_runs_f16_41_v8x1"),
+    # the line: 2^20 vectors
+    ("f32", [64, 256, 255], [0, 2, 1], "permute_runs_f32_64_v4x1"),
+    ("f32", [63, 256, 261], [0, 2, 1], "permute_runs_f32_63_v4x4"),
+    ("f16", [127, 256, 258], [0, 2, 1], "permute_runs_f16_127_v8x1"),
+    ("f16", [127, 256, 259], [0, 2, 1], "permute_runs_f16_127_v8x4"),
+])
+def test_linear_kernel_spreads_small_tensors(host_handle, dtype, lens, perm, name):
+    p = wl.Permutation(host_handle, wl.permutation(dtype, lens, perm))
+    with _Runs():
+        assert p.info()["kernel_name"] == name
+    p.close()
+
+
+class _Runs:
+    """The linear kernel wherever the layout admits it, for the duration of a block."""
+
+    def __enter__(self):
+        os.environ["HIPTENSOR_AMD_PERMUTE"] = "runs"
+
+    def __exit__(self, *a):
+        del os.environ["HIPTENSOR_AMD_PERMUTE"]
 
 
 def test_every_validation_case_plans(host_handle):
