@@ -432,17 +432,30 @@ namespace hipta
             //     229.60.25.24 -> (0,3,2,1) 22.3 -> 10.5, f16 33.500.700.8 -> (0,2,1,3) 430 -> 178;
             //   - the tiles' lanes mostly fall outside: f32 30.7.61.7.7.65 -> (0,4,2,3,1,5) 468 -> 91 (11 % inside),
             //     f16 40.64.128.256 -> (0,3,2,1) 116 -> 77 (31 %), f16 64.64.128.256 -> (0,2,1,3) 104 -> 96, f32
-            //     16.64.128.512 146 -> 130 (50 %; but f32 32.64.128.512, half of a square tile, 198 and 201);
-            //   - or a square tile cuts the run into 256 bytes, which only a tensor beyond the L2 minds: f32
-            //     128.64.128.200 -> (0,2,1,3) 301 -> 270, f16 256.64.128.256 378 -> 347.
-            // Whole runs of full vectors stay in tiles: f32 64.64.64.256 -> (0,3,2,1) 96 against 108,
-            // 256.64.128.128 341 and 347; and so do tensors of a launch's worth of latency (33.40.30 6.4 us on
-            // either, 64.40.30 6.3 and 6.5).
-            const Tile   tt     = (in.elem_bytes == 4 ? TILES4 : TILES2)[out.tile];
+            //     16.64.128.512 146 -> 130 (50 %; but f32 32.64.128.512, half of a square tile, 198 and 201)
+            //   - or a square tile cuts the run into 256 bytes: f32 1140.228.824 -> (0,2,1) 626 -> 298 us, f16 1032.191.1182
+            //     320 -> 149 (150 random shapes: 0.45-1.04, mean 0.64).
+            // Runs of whole 128-byte lines are what tiles do well.  On large tensors (f32 from 2^24, f16 from 2^27 elements)
+            // cut runs of whole lines go linear only where the next runs lie near in A (up to 512 of them at most
+            // 1 MiB apart; f32 128.64.128.200 -> (0,2,1,3) 301 -> 271, f16 256.64.128.256 383 -> 352, both sides level for f32
+            // up to 2^27): far ones make the linear walk read all over the tensor before it comes back to a run's
+            // neighbours, which tiles read together (f32 192.128.2730 -> (0,2,1) 97 us in tiles and 111 linear,
+            // 128.16.1024.64 -> (0,3,2,1) 199 and 251).  Likewise half-empty tiles that are long along the run
+            // (f32 256 x 16 0.79-0.82 of the tiles' time up to 2^22 elements, 0.85-1.42 from 2^24 on; f16
+            // 256.32.1024.32 -> (0,3,2,1) 197 and 240).  Over 400 shapes that this leaves in tiles: linear 0.82-1.42, mean 0.99.
+            // Whole runs of full vectors that tiles cover stay in tiles: f32 64.64.64.256 -> (0,3,2,1) 100 against
+            // 114, 256.64.128.128 347 and 352; and so do tensors that a launch hides on either (33.40.30 4.0 us in
+            // tiles and 2.5 linear, 64.40.30 3.1 and 2.4).
+            const bool   f32    = in.elem_bytes == 4;
+            const Tile   tt     = (f32 ? TILES4 : TILES2)[out.tile];
             const double inside = coverage(ext[0], tt.ti) * coverage(ext[mj], tt.tj);
             const bool   narrow = out.vec_r < full;
-            const bool   sparse = inside <= (in.elem_bytes == 4 && out.tile == 0 ? 0.45 : 0.55);
-            const bool   cut    = out.tile == 0 && ext[0] >= 2 * tt.ti && count >= (1 << 22);
+            const bool   big    = count >= (f32 ? 1 << 24 : 1 << 27) && ext[0] * in.elem_bytes % 128 == 0;
+            const bool   near   = ext[mj] <= 512 && as[mj] * in.elem_bytes <= (1 << 20);
+            const bool   tiled  = out.tile == 1 && big && (f32 || !near); // long tiles: half inside is no loss
+            const bool   sparse = inside <= ((f32 && out.tile == 0) || tiled ? 0.45 : 0.55);
+            const bool   cut    = out.tile == 0 && ext[0] >= 2 * tt.ti && count >= (1 << 22)
+                             && (!big || (count >= (1 << 27) && near));
             if(runs && tune.kernel < 0 && tune.tile < 0 && count >= (1 << 17) && ext[0] * in.elem_bytes >= 64
                && (narrow || sparse || cut))
             {

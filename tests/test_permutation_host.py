@@ -168,6 +168,33 @@ def test_linear_kernel_spreads_small_tensors(host_handle, dtype, lens, perm, nam
     p.close()
 
 
+@pytest.mark.parametrize("dtype,lens,perm,name", [
+    # the runs of a shared fastest mode that square tiles cut: linear on mid-sized tensors ...
+    ("f32", [128, 128, 512], [0, 2, 1], "permute_runs_f32_128_v4x4"),
+    ("f16", [256, 128, 2048], [0, 2, 1], "permute_runs_f16_256_v8x4"),
+    # ... and on the largest, if the next runs lie near in A
+    ("f32", [128, 64, 128, 200], [0, 2, 1, 3], "permute_runs_f32_128_v4x4"),
+    ("f16", [256, 64, 128, 256], [0, 2, 1, 3], "permute_runs_f16_256_v8x4"),
+    # ... and on any where the run is no whole number of 128-byte lines
+    ("f32", [1140, 228, 824], [0, 2, 1], "permute_runs_f32_1140_v4x4"),
+    ("f32", [396, 13, 21, 15, 63], [0, 4, 3, 2, 1], "permute_runs_f32_396_v4x4"),
+    ("f16", [1032, 191, 1182], [0, 2, 1], "permute_runs_f16_1032_v8x4"),
+    ("f32", [132, 134, 300, 42], [0, 3, 2, 1], "permute_runs_f32_132_v4x4"),
+    # tiles where the linear walk loses locality
+    ("f32", [192, 128, 2730], [0, 2, 1], "permute_rows_f32_64x64_r4_w4"),
+    ("f32", [128, 32, 16, 2048], [0, 3, 2, 1], "permute_rows_f32_64x64_r4_w4"),
+    ("f32", [128, 16, 1024, 64], [0, 3, 2, 1], "permute_rows_f32_64x64_r4_w4"),
+    ("f16", [256, 32, 16, 2048], [0, 3, 2, 1], "permute_rows_f16_128x128_r8_w8"),
+    ("f16", [256, 32, 1024, 32], [0, 3, 2, 1], "permute_rows_f16_512x32_r8_w8"),
+    # half of a long tile inside: linear on smaller tensors
+    ("f32", [128, 8, 16, 64], [0, 2, 1, 3], "permute_runs_f32_128_v4x1"),
+    ("f32", [128, 128, 16, 1024], [0, 2, 1, 3], "permute_rows_f32_256x16_r4_w4"),
+    ("f16", [256, 16, 512, 32], [0, 3, 2, 1], "permute_runs_f16_256_v8x4"),
+])
+def test_linear_kernel_or_row_tiles(host_handle, dtype, lens, perm, name):
+    assert _info(host_handle, dtype, lens, perm)["kernel_name"] == name
+
+
 class _Runs:
     """The linear kernel wherever the layout admits it, for the duration of a block."""
 
