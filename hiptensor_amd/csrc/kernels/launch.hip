@@ -3,6 +3,7 @@
 #include <cstdio>
 #include <cstring>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include "contract_h.hpp"
@@ -139,34 +140,45 @@ namespace hiptk
             }
         };
 
-        // Sum of the split-K partials, and the epilogue.  Bound by the latency of its loads, not by their bytes: one thread
-        // per output that walked the slices one load after another took 4-5 us for 8 slices, 9.5 for 32 and 16-20 for
-        // 64, whatever the size of the output.  So a thread owns V consecutive outputs of `per` consecutive slices, has
-        // up to eight of their loads in flight, and looks up where they go beside them; where that leaves the device idle (small outputs, many slices) the
-        // slices are dealt to `groups` threads of the workgroup, whose sums are added up through LDS in slice order.
-        // (64 x 64 outputs in 64 slices: 19.8 -> 3.8 us; 90 x 80 in 32: 9.7 -> 4.1; 256 x 256 in 32: 9.4 -> 4.8.)  The order of
-        // the sum depends on the problem alone: results are the same on every run.
-        template <typename Fin, int V>
-        __global__ void __launch_bounds__(256) splitk_reduce_kernel(const KArgs a, int groups, int per)
+        // Sum of the split-K partials, and the epilogue.  Bound by the latency of its loads where outputs are few, by the
+        // caches and HBM where they are many.  A thread owns V consecutive outputs, has DEPTH slices' loads of them in
+        // flight, takes what is left of its slices in fours, twos and ones (loads repeated to fill a batch cost 0.4 us at two
+        // slices of few outputs and up to 1.2 of many), and looks up where the outputs go beside the loads.  DEALT: where
+        // outputs leave the device idle the slices are dealt to 2^(8 - lane_bits) threads of the workgroup, `per`
+        // consecutive ones each, whose sums are added up through LDS in slice order.  One thread per output that walks
+        // the slices one load after another takes 4-5 us for 8 slices, 9.5 for 32 and 16-20 for 64, whatever the
+        // size of the output; here f32 64 x 64 in 64 slices 3.3 (18.4), 90 x 80 in 32 2.9 (9.5), 256 x 256 in 32 3.4 (9.5), in 2
+        // 2.5 (2.4), 1450 x 1450 in 4 7.3 (10.4), 2048 x 2048 in 2 9.1 (11.3).  Behind it: 16 and more slices of outputs of
+        // 8 or 16 bytes that lie a power of two apart (c32 1024 x 1024 in 16 23.0 and 20.6; the planner cuts no such
+        // output into so many).
+        // The order of the sum depends on the problem alone: results are the same on every run.
+        template <typename Fin, int V, bool DEALT, int DEPTH>
+        __global__ void __launch_bounds__(256) splitk_reduce_kernel(const KArgs a, int lane_bits, int per)
         {
+            static_assert(V == 1 || !DEALT, "dealt slices: one output a thread");
             typedef typename Fin::O O;
             typedef typename Fin::E E;
             struct Vec
             {
                 O v[V];
             };
-            __shared__ Vec part[256];
+            struct Elems
+            {
+                E v[V];
+            };
             const size_t total = (size_t)a.P * (size_t)a.Q;
-            const int    lanes = 256 / groups; // output vectors of this workgroup
-            const int    lane = (int)threadIdx.x % lanes, g = (int)threadIdx.x / lanes;
-            const size_t idx   = ((size_t)blockIdx.x * lanes + lane) * V;
-            const O*     ws    = (const O*)a.ws;
+            const int    lane  = DEALT ? (int)threadIdx.x & ((1 << lane_bits) - 1) : (int)threadIdx.x;
+            const int    g     = DEALT ? (int)threadIdx.x >> lane_bits : 0;
+            const size_t idx   = (((size_t)blockIdx.x << (DEALT ? lane_bits : 8)) + lane) * V;
+            const bool   in    = idx < total;
+            if(!DEALT && !in)
+                return;
             // the last vector starts inside the tensor and may reach beyond it: it is loaded V elements from the end
             // of the slice (which holds more than V), and only its own outputs are kept
-            const bool   in    = idx < total;
-            const int    over  = in && idx + V > total ? (int)(idx + V - total) : 0;
-            const int    z0 = g * per, z1 = z0 + per < a.split_k ? z0 + per : a.split_k;
-            const bool bil = a.bilinear != 0;
+            const int  over = V > 1 && idx + V > total ? (int)(idx + V - total) : 0;
+            const int  z0   = DEALT ? g * per : 0;
+            const int  n    = !DEALT ? a.split_k : !in ? 0 : z0 + per < a.split_k ? per : a.split_k - z0;
+            const bool bil  = a.bilinear != 0;
             // where the outputs go, and their elements of C: looked up beside the partials, not behind them
             // (an output vector may run over the end of a row of D)
             int p, q;
@@ -182,11 +194,7 @@ namespace hiptk
             }
             uint32_t doff[V], coff[V];
             bool     d_run = idx + V <= total, c_run = d_run; // one run of V elements of D / C
-            struct Elems
-            {
-                E v[V];
-            };
-            Elems c = {};
+            Elems    c     = {};
 #pragma unroll
             for(int e = 0; e < V; e++)
             {
@@ -221,56 +229,52 @@ namespace hiptk
                         c.v[e] = ((const E*)a.C)[coff[e]];
                 }
             }
-            Vec          s = {};
-            auto         add = [&](const Vec& x) {
+            const O* src = (const O*)a.ws + (size_t)z0 * total + (idx - over);
+            Vec      s   = {};
+            auto     add = [&](const Vec& x) {
 #pragma unroll
                 for(int e = 0; e < V; e++)
                     s.v[e] = Fin::add(s.v[e], x.v[e]);
             };
-            if(in && z0 < z1)
+            auto take = [&](auto width, int z) {
+                constexpr int W = decltype(width)::value;
+                Vec           x[W];
+#pragma unroll
+                for(int u = 0; u < W; u++)
+                    __builtin_memcpy(&x[u], src + (size_t)(z + u) * total, sizeof(Vec));
+                if(z == 0)
+                    s = x[0];
+                else
+                    add(x[0]);
+#pragma unroll
+                for(int u = 1; u < W; u++)
+                    add(x[u]);
+            };
+            int z = 0;
+            for(; z + DEPTH <= n; z += DEPTH)
+                take(std::integral_constant<int, DEPTH>{}, z);
+            if(DEPTH > 4 && z + 4 <= n) // (fewer than DEPTH are left)
             {
-                const O* src = ws + (size_t)z0 * total + (idx - over);
-                auto     load = [&](int z) {
-                    Vec x;
-                    __builtin_memcpy(&x, src + (size_t)z * total, sizeof(x));
-                    return x;
-                };
-                s     = load(0);
-                int z = 1;
-                for(; z + 8 <= z1 - z0; z += 8)
-                {
-                    Vec x[8];
-#pragma unroll
-                    for(int u = 0; u < 8; u++)
-                        x[u] = load(z + u);
-#pragma unroll
-                    for(int u = 0; u < 8; u++)
-                        add(x[u]);
-                }
-                if(z < z1 - z0)
-                {
-                    // (the rest, the loads beyond it repeating the last slice)
-                    Vec x[7];
-#pragma unroll
-                    for(int u = 0; u < 7; u++)
-                        x[u] = load(z + u < z1 - z0 ? z + u : z1 - z0 - 1);
-#pragma unroll
-                    for(int u = 0; u < 7; u++)
-                        if(z + u < z1 - z0)
-                            add(x[u]);
-                }
+                take(std::integral_constant<int, 4>{}, z);
+                z += 4;
             }
-            if(groups > 1)
+            if(z + 2 <= n)
             {
+                take(std::integral_constant<int, 2>{}, z);
+                z += 2;
+            }
+            if(z < n)
+                take(std::integral_constant<int, 1>{}, z);
+            if constexpr(DEALT)
+            {
+                __shared__ Vec part[256];
                 part[threadIdx.x] = s;
                 __syncthreads();
-                if(g != 0)
+                if(g != 0 || !in)
                     return;
-                for(int h = 1; h < groups && h * per < a.split_k; h++)
-                    add(part[h * lanes + lane]);
+                for(int h = 1; h < 256 >> lane_bits && h * per < a.split_k; h++)
+                    add(part[(h << lane_bits) + lane]);
             }
-            if(!in)
-                return;
             // the last vector's outputs back to the front
 #pragma unroll
             for(int h = 1; h < V; h++)
@@ -295,29 +299,35 @@ namespace hiptk
             }
         }
 
-        template <typename Fin, int V>
-        int launch_reduce_v(const KArgs& a, hipStream_t stream)
-        {
-            const size_t vecs = ((size_t)a.P * (size_t)a.Q + V - 1) / V;
-            // threads enough for 16 wavefronts a compute unit, at least four slices each
-            int groups = 1;
-            while(groups < 32 && vecs * (size_t)groups < 131072 && a.split_k / (2 * groups) >= 4)
-                groups *= 2;
-            const int    per    = (a.split_k + groups - 1) / groups;
-            const size_t lanes  = 256 / (size_t)groups;
-            const size_t blocks = (vecs + lanes - 1) / lanes;
-            hipLaunchKernelGGL((splitk_reduce_kernel<Fin, V>), dim3((unsigned)blocks), dim3(256), 0, stream, a, groups, per);
-            return (int)hipGetLastError();
-        }
-
         template <typename Fin>
         int launch_reduce(const KArgs& a, hipStream_t stream)
         {
-            constexpr int V = sizeof(typename Fin::O) >= 16 ? 1 : 16 / (int)sizeof(typename Fin::O);
-            // 16 bytes a thread once that still puts eight wavefronts on every compute unit; one output below
-            if((size_t)a.P * (size_t)a.Q >= (size_t)V * 131072)
-                return launch_reduce_v<Fin, V>(a, stream);
-            return launch_reduce_v<Fin, 1>(a, stream);
+            constexpr int V     = sizeof(typename Fin::O) >= 16 ? 1 : 16 / (int)sizeof(typename Fin::O);
+            const size_t  total = (size_t)a.P * (size_t)a.Q;
+            // 16 bytes a thread once that still puts eight wavefronts on every compute unit, if the outputs are one run of
+            // D after another (f32 1450 x 1450 in 4 slices 7.3 us, one output a thread 8.4; with offsets from tables, of
+            // which a thread then has V to wait for, 2048 x 2048 in 2 17.4 and 14.2)
+            if(V > 1 && total >= (size_t)V * 131072 && a.cd_affine && a.dq_stride == 1)
+            {
+                const size_t blocks = (total + 256 * V - 1) / (256 * V);
+                hipLaunchKernelGGL((splitk_reduce_kernel<Fin, V, false, 4>), dim3((unsigned)blocks), dim3(256), 0, stream, a, 8, a.split_k);
+                return (int)hipGetLastError();
+            }
+            // four 16-byte loads or eight smaller ones in flight: more from slices that lie a power of two apart meet in the
+            // same channels (f32 1024 x 1024 in 16 slices 12.3 us against 13.6 with eight of 16 bytes, c64 512 x 512 in 16
+            // 11.9 and 13.4), fewer wait (f32 700 x 750 in 16, four of 4 bytes 8.0, eight 6.8)
+            constexpr int DEPTH = sizeof(typename Fin::O) >= 16 ? 4 : 8;
+            // threads enough for eight wavefronts a compute unit, at least four slices each
+            int lane_bits = 8;
+            while(lane_bits > 3 && (total << (8 - lane_bits)) < 131072 && (a.split_k >> (9 - lane_bits)) >= 4)
+                lane_bits--;
+            const int    groups = 256 >> lane_bits, per = (a.split_k + groups - 1) / groups;
+            const size_t blocks = (total + ((size_t)1 << lane_bits) - 1) >> lane_bits;
+            if(groups > 1)
+                hipLaunchKernelGGL((splitk_reduce_kernel<Fin, 1, true, DEPTH>), dim3((unsigned)blocks), dim3(256), 0, stream, a, lane_bits, per);
+            else
+                hipLaunchKernelGGL((splitk_reduce_kernel<Fin, 1, false, DEPTH>), dim3((unsigned)blocks), dim3(256), 0, stream, a, lane_bits, per);
+            return (int)hipGetLastError();
         }
 
         int reduce_dispatch(int cls, const KArgs& a, hipStream_t stream)

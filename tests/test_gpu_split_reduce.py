@@ -19,13 +19,14 @@ TILES = {"f16": (2, 4), "bf16": (2, 4), "f32": (1,), "f64": (1,), "c32": (1,), "
 OUTPUTS = [((1,), (1,)), ((1,), (3,)), ((7,), (9,)), ((13, 10), (67,)), ((29, 25), (726,))]
 
 
-def _run(handle, w, inp, split):
+def _run(handle, w, inp, split, d_alias_c=False):
     """On the first of the class's small tiles that takes the layout."""
     for tile in TILES[w["dtype"]]:
         os.environ["HIPTENSOR_AMD_FORCE_KERNEL"] = f"{tile},{split}"
         print(f"[case] {w['name']} tile={tile} split={split} beta={w['beta']}", flush=True)
         try:
-            return gpu_util.run_gpu(handle, w, inp, pref=api.HIPTENSOR_WORKSPACE_MAX, return_info=True)
+            return gpu_util.run_gpu(handle, w, inp, pref=api.HIPTENSOR_WORKSPACE_MAX, d_alias_c=d_alias_c,
+                                    return_info=True)
         except api.HiptensorError as e:
             assert e.status == api.HIPTENSOR_STATUS_EXECUTION_FAILED and tile != TILES[w["dtype"]][-1], e
         finally:
@@ -52,3 +53,45 @@ def test_reduction_forms(gpu_handle, oracle_mod, dtype, m, n):
                 got, info = _run(gpu_handle, w, inp, split)
                 assert info["split_k"] == split
                 cases.assert_parity(w, cases.logical_view(w, got), exp, f"{info['kernel_name']} split {split}")
+
+
+# largest K tile of the tiles above
+K_TILE = {"f16": 64, "bf16": 64, "f32": 16, "f64": 16, "c32": 8, "c64": 8}
+
+
+def _one(handle, oracle_mod, dtype, m, n, k_tiles, split, beta, table=False, alias=False):
+    k = k_tiles * K_TILE[dtype]
+    a = 1.1 + 0.4j if dtype.startswith("c") else 1.5
+    b = None if not beta else 0.6 - 0.3j if dtype.startswith("c") else 0.75
+    modes = list(range(len(m))), list(range(10, 10 + len(n)))
+    ext = {**dict(zip(modes[0], m)), **dict(zip(modes[1], n)), 20: k}
+    d = modes[0] + modes[1]
+    w = wl.make_workload(dtype, cases.COMPUTE[dtype], modes[0] + [20], modes[1] + [20], d[::-1] if table else d, ext, a, b,
+                         name=f"reduce_{dtype}_{'x'.join(map(str, m))}_{'x'.join(map(str, n))}_{k}")
+    inp = wl.host_inputs(w)
+    exp = cases.logical_view(w, oracle_mod.contract(w, inp["A"], inp["B"], inp["C"]))
+    got, info = _run(handle, w, inp, split, d_alias_c=alias)
+    assert info["split_k"] == split
+    tiles = k // info["tile_k"]
+    slices = -(-tiles // -(-tiles // split))  # none of them empty
+    assert slices > 8 and slices % 4 != 0, info
+    cases.assert_parity(w, cases.logical_view(w, got), exp, f"{info['kernel_name']} split {split}")
+
+
+@pytest.mark.parametrize("dtype", list(TILES))
+@pytest.mark.parametrize("m,n,table", [((7,), (9,), False), ((16, 16), (16, 16), False), ((16, 17), (241,), True), ((400,), (331,), False)])
+def test_many_slices(gpu_handle, oracle_mod, dtype, m, n, table):
+    """A hundred K tiles in 32 and 64 slices asked for: 25 and 50 slices of four and two tiles, so that the threads of a
+    workgroup get unequal numbers of them, and a thread has whole batches of loads and a rest."""
+    for split in (32, 64):
+        for beta in (False, True):
+            _one(gpu_handle, oracle_mod, dtype, m, n, 100, split, beta, table)
+
+
+@pytest.mark.parametrize("dtype", list(TILES))
+@pytest.mark.parametrize("m,n", [((725,), (725,)), ((29, 25), (726,)), ((29, 25), (11, 66)), ((1100,), (500,))])
+def test_large_outputs(gpu_handle, oracle_mod, dtype, m, n):
+    """16 bytes of outputs a thread and eleven slices (two batches of four and a rest); 1, 2, 2 and 0 outputs left behind the
+    last whole vector; D apart from C and in its place, computed offsets and ones from tables (rows along D and across it)."""
+    for beta, table, alias in ((False, False, False), (True, False, True), (True, True, True)):
+        _one(gpu_handle, oracle_mod, dtype, m, n, 22, 16, beta, table, alias)
