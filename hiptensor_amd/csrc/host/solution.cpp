@@ -302,9 +302,16 @@ namespace hipta
             // partials out and back, second launch; partials that fit the 256 MiB last-level
             // cache never reach HBM
             const double bw = ws <= 160e6 ? dev.hbm_gbs * 1e3 * 1.0 : dev.hbm_gbs * 1e3 * 0.6;
-            // the reduction walks the slices one after another; and short slices are mostly prologue
-            // (512^3 in 8 slices against 4: f32 14.0 / 11.9 us, complex f32 24.5 / 20.5, 256^3 complex f64 13.5 / 11.3)
-            us += 2.0 * ws / bw + 3.0 + 0.25 * split;
+            // the reduction's launch, and the prologue of more and shorter slices (8 against 4, the reduction of both alike:
+            // 512^3 f32 12.9 / 11.1 us, 256^3 complex f64 12.8 / 10.6).  The reduction takes 2.5 us of two slices and 3.4 of
+            // 64, so what more than 16 of them add is prologue alone, and little while they have K tiles enough (f16
+            // 199 x 191 x 94385 in 64 slices of 128 x 128 tiles 41 us, in 32 of 64 x 64 57; f32 104 x 34 x 10880 where
+            // it lies in 64 12.1, packed and in 16 19.6).  Over 570 shapes the choice takes 1.03 of the time of the best
+            // tile and split (1.06 with 0.25 a slice throughout).
+            double per_slice = 0.25 * split;
+            if(split > 16)
+                per_slice = std::min(per_slice, 4.0 + 0.05 * (split - 16) + 0.2 * std::max(0.0, 16.0 - kper / s.bk));
+            us += 2.0 * ws / bw + 3.0 + per_slice;
         }
         return us;
     }

@@ -246,3 +246,19 @@ def test_direct_load_kernels_keep_32_bit_offsets_in_range(host_handle, monkeypat
             assert (name is not None and "direct" in name) == offered, (stride, force, name)
         name = kernel(stride, None)
         assert name is not None and (offered or "direct" not in name), (stride, name)
+
+
+@pytest.mark.parametrize("dtype,modes,ext,split,packed", [
+    # small results of long reductions: the slices' reduction costs about a microsecond more for 64 of them than for two
+    ("f16", ([0, 20], [20, 10], [0, 10]), {0: 199, 10: 191, 20: 94385}, 64, 0),
+    ("f32", ([20, 21, 0], [20, 10, 21], [0, 10]), {0: 104, 10: 34, 20: 34, 21: 320}, 64, 0),
+    ("f64", ([20, 0], [20, 10], [10, 0]), {0: 55, 10: 173, 20: 9726}, 64, 0),
+    ("bf16", ([20, 0], [20, 10], [10, 0]), {0: 36, 10: 216, 20: 36540}, 64, 0),
+    # ... but slices of few K tiles are mostly prologue
+    ("f16", ([0, 20], [10, 20], [0, 10]), {0: 160, 10: 160, 20: 2048}, 8, 0),
+    ("f32", ([0, 20], [10, 20], [0, 10]), {0: 256, 10: 256, 20: 256}, 1, 0),
+])
+def test_slices_of_long_reductions(host_handle, dtype, modes, ext, split, packed):
+    w = wl.make_workload(dtype, cases.COMPUTE[dtype], *modes, ext, 1.5, None, name="long_k")
+    info, _ = plan(host_handle, w)
+    assert (info["split_k"], info["pack_a"] + info["pack_b"]) == (split, packed), info["kernel_name"]
