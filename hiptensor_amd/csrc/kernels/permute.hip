@@ -35,13 +35,12 @@
 #include <type_traits>
 
 #include "hiptk_kernels.h"
+#include "perm_addr.hpp"
 
 namespace hiptk
 {
     namespace
     {
-        constexpr int PERM_THREADS = 256;
-        constexpr int PERM_BATCH   = HIPTK_PERM_MAX_RANK - 2;
 
         struct PArgs
         {
@@ -435,25 +434,11 @@ namespace hiptk
             }
         }
 
-        // 2^32 / d rounded up, d >= 2: __umulhi(v, recip(d)) == v / d while v * d < 2^32
-        __device__ inline uint32_t recip(uint32_t d)
-        {
-            return 0xFFFFFFFFu / d + 1u;
-        }
-
         struct QArgs
         {
+            GroupShape  s;
             const void* A;
             void*       B;
-            uint32_t    e_i0, e_i1, e_j0, e_j1; // extents of the row modes (0, i2) and the column modes (j, j2); 1 if absent
-            uint32_t    w_i, w_j; // elements of mode 0 / mode j per tile (== the extent when c > 1)
-            uint32_t    c_i, c_j; // indices of i2 / j2 per tile
-            uint32_t    a_j0, a_j1, b_i0, b_i1; // A strides of the column modes, B strides of the row modes
-            uint32_t    nt_i0, nt_j0, nt_i, nt_j; // tiles along mode 0, mode j, i2 and j2
-            uint32_t    pitch; // LDS row pitch in elements: an odd number of 32-bit words
-            uint32_t    m_rv, m_wj, m_cv, m_wi; // floor(2^32 / d) + 1 for d = TI / VR, w_j, TJ / VW, w_i
-            int32_t     nb;
-            uint32_t    bext[PERM_BATCH], ba[PERM_BATCH], bb[PERM_BATCH];
             float       alpha;
             int32_t     op_a, op_b;
         };
@@ -481,40 +466,13 @@ namespace hiptk
             T* __restrict__ B       = static_cast<T*>(a.B);
             const uint32_t tid      = threadIdx.x;
 
-            uint32_t       blk = blockIdx.x;
-            const uint32_t ti0 = blk % a.nt_i0;
-            blk /= a.nt_i0;
-            const uint32_t tj0 = blk % a.nt_j0;
-            blk /= a.nt_j0;
-            const uint32_t ti = blk % a.nt_i;
-            blk /= a.nt_i;
-            const uint32_t tj = blk % a.nt_j;
-            blk /= a.nt_j;
-            uint32_t aoff = 0, boff = 0;
-            for(int d = 0; d < a.nb; ++d)
-            {
-                const uint32_t c = blk % a.bext[d];
-                blk /= a.bext[d];
-                aoff += c * a.ba[d];
-                boff += c * a.bb[d];
-            }
-            const uint32_t i0s = ti0 * a.w_i, j0s = tj0 * a.w_j;
-            const uint32_t wi = (a.e_i0 - i0s) < a.w_i ? (a.e_i0 - i0s) : a.w_i;
-            const uint32_t wj = (a.e_j0 - j0s) < a.w_j ? (a.e_j0 - j0s) : a.w_j;
-            const uint32_t i1s = ti * a.c_i, j1s = tj * a.c_j;
-            const uint32_t ci = (a.e_i1 - i1s) < a.c_i ? (a.e_i1 - i1s) : a.c_i;
-            const uint32_t cj = (a.e_j1 - j1s) < a.c_j ? (a.e_j1 - j1s) : a.c_j;
-            // rows and columns inside the extents (c > 1 only with the whole first mode: w == e)
-            const uint32_t nx = a.w_i * (ci - 1) + wi, ny = a.w_j * (cj - 1) + wj;
-            // vectors per nominal row / column
-            const uint32_t RV = (a.w_i * a.c_i + (LOOSE ? VR - 1 : 0)) / VR, CV = (a.w_j * a.c_j + (LOOSE ? VW - 1 : 0)) / VW;
-            aoff += i0s + i1s * a.e_i0 + j0s * a.a_j0 + j1s * a.a_j1;
-            boff += i0s * a.b_i0 + i1s * a.b_i1 + j0s + j1s * a.e_j0;
-            const T alpha = static_cast<T>(a.alpha);
+            const GroupTile t     = group_tile(a.s, blockIdx.x);
+            const uint32_t  RV    = group_per_line(a.s.w_i * a.s.c_i, VR, LOOSE), CV = group_per_line(a.s.w_j * a.s.c_j, VW, LOOSE);
+            const T         alpha = static_cast<T>(a.alpha);
 
             auto read = [&](auto width, uint32_t per_row, uint32_t m_row) {
                 constexpr int  W     = decltype(width)::value;
-                const uint32_t total = per_row * ny;
+                const uint32_t total = per_row * t.ny;
                 for(uint32_t u0 = 0; u0 < total; u0 += NT * U)
                 {
                     Vec<T, W> r[U];
@@ -522,16 +480,10 @@ namespace hiptk
 #pragma unroll
                     for(int k = 0; k < U; ++k)
                     {
-                        const uint32_t v  = u0 + tid + k * NT;
-                        const uint32_t y  = __umulhi(v, m_row);
-                        uint32_t       x  = (v - y * per_row) * W;
-                        const uint32_t y1 = __umulhi(y, a.m_wj), y0 = y - y1 * a.w_j;
-                        const bool     ok = v < total && x < nx;
-                        if constexpr(LOOSE)
-                            x = x + W > nx ? nx - W : x;
-                        at[k] = ok ? y * a.pitch + x : 0xFFFFFFFFu;
+                        const GroupVector g = group_read<W, LOOSE>(a.s, t, u0 + tid + k * NT, per_row, m_row);
+                        at[k]               = g.ok ? g.line * a.s.pitch + g.at : 0xFFFFFFFFu;
                         // out-of-range lanes load the tile's first element: no branch, all loads in flight
-                        const T* from = A + aoff + (ok ? x + y0 * a.a_j0 + y1 * a.a_j1 : 0u);
+                        const T* from = A + t.aoff + (g.ok ? g.at + g.off : 0u);
                         if constexpr(LOOSE && W > 1)
                             r[k] = load_loose(from);
                         else
@@ -551,21 +503,17 @@ namespace hiptk
             };
             auto write = [&](auto width, uint32_t per_col, uint32_t m_col) {
                 constexpr int  W     = decltype(width)::value;
-                const uint32_t total = per_col * nx;
+                const uint32_t total = per_col * t.nx;
                 for(uint32_t v = tid; v < total; v += NT)
                 {
-                    const uint32_t x = __umulhi(v, m_col);
-                    uint32_t       y = (v - x * per_col) * W;
-                    if(y < ny)
+                    const GroupVector g = group_write<W, LOOSE>(a.s, t, v, per_col, m_col);
+                    if(g.ok)
                     {
-                        if constexpr(LOOSE)
-                            y = y + W > ny ? ny - W : y;
-                        const uint32_t x1 = __umulhi(x, a.m_wi), x0 = x - x1 * a.w_i;
-                        Vec<T, W>      o;
+                        Vec<T, W> o;
 #pragma unroll
                         for(int e = 0; e < W; ++e)
-                            o.v[e] = tile[(y + e) * a.pitch + x];
-                        T* to = B + boff + y + x0 * a.b_i0 + x1 * a.b_i1;
+                            o.v[e] = tile[(g.at + e) * a.s.pitch + g.line];
+                        T* to = B + t.boff + g.at + g.off;
                         if constexpr(LOOSE && W > 1)
                             store_loose(to, o);
                         else
@@ -574,15 +522,15 @@ namespace hiptk
                 }
             };
             typedef std::integral_constant<int, 1> One;
-            if(!LOOSE || nx >= VR)
-                read(std::integral_constant<int, VR>{}, RV, a.m_rv);
+            if(!LOOSE || t.nx >= VR)
+                read(std::integral_constant<int, VR>{}, RV, a.s.m_rv);
             else
-                read(One{}, nx < 2 ? 2 : nx, recip(nx < 2 ? 2 : nx));
+                read(One{}, group_singles(t.nx), recip(group_singles(t.nx)));
             __syncthreads();
-            if(!LOOSE || ny >= VW)
-                write(std::integral_constant<int, VW>{}, CV, a.m_cv);
+            if(!LOOSE || t.ny >= VW)
+                write(std::integral_constant<int, VW>{}, CV, a.s.m_cv);
             else
-                write(One{}, ny < 2 ? 2 : ny, recip(ny < 2 ? 2 : ny));
+                write(One{}, group_singles(t.ny), recip(group_singles(t.ny)));
         }
 
         struct HArgs
@@ -736,29 +684,12 @@ namespace hiptk
 
         struct RArgs
         {
+            RunsShape   s;
             const void* A;
             void*       B;
-            uint32_t    n; // elements
-            uint32_t    e0, m0; // extent of the shared fastest mode and its reciprocal
-            int32_t     nb; // the other modes, in B's order
-            uint32_t    ext[HIPTK_PERM_MAX_RANK - 1], astr[HIPTK_PERM_MAX_RANK - 1], magic[HIPTK_PERM_MAX_RANK - 1];
             float       alpha;
             int32_t     op_a, op_b;
         };
-
-        // x / e and x % e by the reciprocal m = floor(2^32 / e) + 1, exact for every 32-bit x (the high word is the
-        // quotient or one more)
-        __device__ inline uint32_t div_by(uint32_t x, uint32_t e, uint32_t m, uint32_t& rem)
-        {
-            uint32_t q = __umulhi(x, m), r = x - q * e;
-            if((int32_t)r < 0)
-            {
-                q -= 1;
-                r += e;
-            }
-            rem = r;
-            return q;
-        }
 
         // A and B share the fastest mode, of V = 16 bytes' worth of elements or more.  Bound by HBM.  A tile of two modes
         // wastes the lanes that overhang them, and needs vectors that divide the run; here a vector is any V consecutive
@@ -766,7 +697,7 @@ namespace hiptk
         // and stores at any multiple of the element), or in two where the vector spans the end of a run.
         // f32 21.79.79.20.8.7 -> (0,1,3,4,5,2), 587 MB: 443 us in tiles, 203 here (5.8 TB/s); f32 30.7.61.7.7.65 ->
         // (0,4,2,3,1,5), 163 MB in runs of 120 bytes: 468 -> 91 us (3.6 TB/s: the run's ends share lines with others').
-        // A thread moves U vectors, its loads all in flight.
+        // A thread moves U vectors, both loads of each in flight with the others'.
         template <typename T, int U>
         __global__ __launch_bounds__(PERM_THREADS) void permute_runs_kernel(RArgs a)
         {
@@ -777,72 +708,39 @@ namespace hiptk
             const T alpha           = static_cast<T>(a.alpha);
             auto    load            = [&](uint32_t off) { return load_loose(A + off); };
 
-            const uint32_t last  = a.n - V; // the last vector is moved back to end with the tensor
+            const uint32_t last  = a.s.n - V; // the last vector is moved back to end with the tensor
             const uint32_t first = (blockIdx.x * (PERM_THREADS * U) + threadIdx.x) * V;
-            uint32_t       src[U], next[U], left[U]; // the vector's place in A, that of its next run, elements of this run from it on
-            Elems          x[U];
+            RunsVector     r[U];
+            Elems          x[U], y[U];
 #pragma unroll
             for(int u = 0; u < U; ++u)
             {
-                const uint32_t at  = first + u * PERM_THREADS * V;
-                const uint32_t idx = at < last ? at : last;
-                uint32_t       pos, off = 0, noff = 0;
-                uint32_t       rem   = div_by(idx, a.e0, a.m0, pos);
-                bool           carry = true; // the next run's coordinates: one more, from the fastest mode up
-                for(int d = 0; d < a.nb; ++d)
-                {
-                    uint32_t c;
-                    rem = div_by(rem, a.ext[d], a.magic[d], c);
-                    const uint32_t c1 = !carry ? c : c + 1 == a.ext[d] ? 0u : c + 1;
-                    off += c * a.astr[d];
-                    noff += c1 * a.astr[d];
-                    carry = carry && c1 == 0;
-                }
-                src[u]  = off + pos;
-                next[u] = noff;
-                left[u] = a.e0 - pos;
-                x[u]    = load(src[u] < last ? src[u] : last);
+                const uint32_t at = first + u * PERM_THREADS * V;
+                r[u]              = runs_vector(a.s, at < last ? at : last);
+                x[u]              = load(r[u].src);
+                if(r[u].left < V)
+                    y[u] = load(r[u].next - r[u].left);
             }
 #pragma unroll
             for(int u = 0; u < U; ++u)
             {
-                if(left[u] < V)
+                const uint32_t k = r[u].left;
+                if(k < V)
                 {
-                    const uint32_t k = left[u];
-                    if(src[u] <= last && next[u] >= k)
-                    {
-                        const Elems y = load(next[u] - k);
 #pragma unroll
-                        for(int e = 1; e < V; ++e)
-                            x[u].v[e] = (uint32_t)e < k ? x[u].v[e] : y.v[e];
-                    }
-                    else // one of the two vectors would reach beyond the ends of A
-                    {
-#pragma unroll
-                        for(int e = 0; e < V; ++e)
-                            x[u].v[e] = A[(uint32_t)e < k ? src[u] + e : next[u] + (e - k)];
-                    }
+                    for(int e = 1; e < V; ++e)
+                        x[u].v[e] = (uint32_t)e < k ? x[u].v[e] : y[u].v[e];
                 }
                 const uint32_t at = first + u * PERM_THREADS * V;
 #pragma unroll
                 for(int e = 0; e < V; ++e)
                     x[u].v[e] = element_op(x[u].v[e], alpha, a.op_a, a.op_b);
-                if(at < a.n)
+                if(at < a.s.n)
                     store_loose(B + (at < last ? at : last), x[u]);
             }
         }
 
         // ---------------------------------------------------------------- host side
-
-        // Vectors per thread of the RUNS kernel.  Four keep more loads in flight, but a tensor of a few MB then makes too few
-        // workgroups for 256 compute units and the kernel lasts as long as one thread (2^17 f32: 32 workgroups): f32
-        // 16.20.4.8.8.4 -> (0,1,4,3,5,2) 5.7 us, 3.9 in tiles; one per thread takes 0.58-0.75 of four's time up to 2^20
-        // f32 (0.60-0.72 up to 2^21 f16), 0.87-0.91 just below the line here and 0.94-1.02 beyond it, with cases of up
-        // to 1.24.  From four workgroups of four a compute unit on, four.
-        int runs_per_thread(int64_t n, int v)
-        {
-            return n >= (int64_t(1) << 20) * v ? 4 : 1;
-        }
 
         struct TileShape
         {
@@ -971,11 +869,6 @@ namespace hiptk
 
         constexpr int GROUP_MAX_FAST = 128; // longest fastest mode the grouped kernel takes
         constexpr int GROUP_MAX_LDS  = 60 * 1024;
-
-        uint32_t magic_of(uint32_t d)
-        {
-            return (uint32_t)((uint64_t(1) << 32) / d) + 1u;
-        }
 
         template <typename T, int VMAX>
         int launch_group(int vr, int vw, bool loose, const QArgs& a, uint32_t grid, size_t lds, hipStream_t s)
@@ -1232,28 +1125,10 @@ extern "C" int hiptk_permute(const hiptk_permute_t* p, const void* A, void* B, v
         memset(&a, 0, sizeof(a));
         a.A     = A;
         a.B     = B;
-        a.n     = (uint32_t)n;
-        a.e0    = (uint32_t)p->extent[0];
-        a.m0    = magic_of(a.e0);
+        a.s     = runs_shape(*p, n);
         a.alpha = p->alpha;
         a.op_a  = p->op_a;
         a.op_b  = p->op_b;
-        int order[HIPTK_PERM_MAX_RANK];
-        for(int d = 0; d < p->rank; ++d)
-            order[d] = d;
-        std::sort(order + 1, order + p->rank, [p](int x, int y) {
-            return p->b_stride[x] != p->b_stride[y] ? p->b_stride[x] < p->b_stride[y] : x < y;
-        });
-        for(int k = 1; k < p->rank; ++k)
-        {
-            const int d = order[k];
-            if(p->extent[d] == 1)
-                continue;
-            a.ext[a.nb]   = (uint32_t)p->extent[d];
-            a.astr[a.nb]  = (uint32_t)p->a_stride[d];
-            a.magic[a.nb] = magic_of((uint32_t)p->extent[d]);
-            ++a.nb;
-        }
         const int      u    = runs_per_thread(n, v);
         const int64_t  per  = (int64_t)PERM_THREADS * u * v;
         const uint32_t grid = (uint32_t)((n + per - 1) / per);
@@ -1372,49 +1247,16 @@ extern "C" int hiptk_permute(const hiptk_permute_t* p, const void* A, void* B, v
         memset(&a, 0, sizeof(a));
         a.A    = A;
         a.B    = B;
-        a.e_i0 = (uint32_t)p->extent[0];
-        a.e_i1 = (uint32_t)e_i1;
-        a.e_j0 = (uint32_t)p->extent[mj];
-        a.e_j1 = (uint32_t)e_j1;
-        a.w_i  = (uint32_t)w_i;
-        a.w_j  = (uint32_t)w_j;
-        a.c_i  = (uint32_t)p->chunk_i;
-        a.c_j  = (uint32_t)p->chunk_j;
-        a.a_j0 = (uint32_t)p->a_stride[mj];
-        a.a_j1 = mj2 == -1 ? 0u : (uint32_t)p->a_stride[mj2];
-        a.b_i0 = (uint32_t)p->b_stride[0];
-        a.b_i1 = mi2 == -1 ? 0u : (uint32_t)p->b_stride[mi2];
-        a.nt_i0 = (a.e_i0 + a.w_i - 1) / a.w_i;
-        a.nt_j0 = (a.e_j0 + a.w_j - 1) / a.w_j;
-        a.nt_i  = (a.e_i1 + a.c_i - 1) / a.c_i;
-        a.nt_j  = (a.e_j1 + a.c_j - 1) / a.c_j;
-        const uint32_t TI = a.w_i * a.c_i, TJ = a.w_j * a.c_j;
-        const uint32_t wordElems = 4u / (uint32_t)p->elem_bytes; // elements per 32-bit word
-        uint32_t       pitchWords = (TI + wordElems - 1) / wordElems;
-        pitchWords |= 1u; // odd: consecutive rows start in different banks
-        a.pitch          = pitchWords * wordElems;
-        const size_t lds = (size_t)TJ * a.pitch * p->elem_bytes;
-        if(lds > (size_t)GROUP_MAX_LDS || TI / vr < 2 || TJ / vw < 2 || w_i < 2 || w_j < 2)
-            return HIPTK_ERR_ARG; // (the reciprocals below are exact for divisors of 2 and more)
-        a.m_rv = magic_of(loose ? (TI + vr - 1) / vr : TI / vr);
-        a.m_wj = magic_of(a.w_j);
-        a.m_cv = magic_of(loose ? (TJ + vw - 1) / vw : TJ / vw);
-        a.m_wi = magic_of(a.w_i);
-        a.alpha = p->alpha;
-        a.op_a  = p->op_a;
-        a.op_b  = p->op_b;
-        int64_t grid = (int64_t)a.nt_i0 * a.nt_j0 * a.nt_i * a.nt_j;
-        for(int d = 1; d < p->rank; ++d)
-        {
-            if(d == mj || d == mi2 || d == mj2)
-                continue;
-            a.bext[a.nb] = (uint32_t)p->extent[d];
-            a.ba[a.nb]   = (uint32_t)p->a_stride[d];
-            a.bb[a.nb]   = (uint32_t)p->b_stride[d];
-            ++a.nb;
-            grid *= p->extent[d];
-        }
-        if(grid >= (int64_t(1) << 31))
+        const uint32_t TI = (uint32_t)w_i * (uint32_t)p->chunk_i, TJ = (uint32_t)w_j * (uint32_t)p->chunk_j;
+        if(TI / vr < 2 || TJ / vw < 2 || w_i < 2 || w_j < 2)
+            return HIPTK_ERR_ARG; // (the reciprocals are exact for divisors of 2 and more)
+        int64_t grid = 0;
+        a.s          = group_shape(*p, grid);
+        a.alpha      = p->alpha;
+        a.op_a       = p->op_a;
+        a.op_b       = p->op_b;
+        const size_t lds = (size_t)TJ * a.s.pitch * p->elem_bytes;
+        if(lds > (size_t)GROUP_MAX_LDS || grid >= (int64_t(1) << 31))
             return HIPTK_ERR_ARG;
         rc = p->elem_bytes == 4 ? launch_group<float, 4>(vr, vw, loose, a, (uint32_t)grid, lds, s)
                                 : launch_group<_Float16, 8>(vr, vw, loose, a, (uint32_t)grid, lds, s);

@@ -5,6 +5,9 @@ from hiptensor_amd import api
 from hiptensor_amd import workloads as wl
 
 
+GUARD_BYTES = 256  # on either side of a permutation's B: more than any vector, and B's alignment with it
+
+
 def to_device(buf):
     import torch
 
@@ -41,7 +44,8 @@ def run_gpu(handle, w, inp=None, algo=api.HIPTENSOR_ALGO_DEFAULT, pref=api.HIPTE
 def run_gpu_permutation(handle, w, A=None, a_shift=0, b_shift=0, return_info=False):
     """Runs one permutation workload; returns packed B as a host array of the storage type.
     a_shift / b_shift move the two device tensors off their allocation's alignment by that
-    many elements.  B is pre-filled with NaN, so an element left unwritten shows."""
+    many elements.  B is pre-filled with NaN, so an element left unwritten shows, and lies between
+    guards that no store may touch."""
     import torch
 
     if A is None:
@@ -51,13 +55,18 @@ def run_gpu_permutation(handle, w, A=None, a_shift=0, b_shift=0, return_info=Fal
     item = np.dtype(t).itemsize
     hostA = np.concatenate([np.zeros(a_shift, dtype=t), np.ascontiguousarray(A, dtype=t)])
     dA = to_device(hostA)
-    dB = to_device(wl.nan_buffer(w["dtype"], n + b_shift))
+    front = GUARD_BYTES // item + b_shift
+    guard = np.full(GUARD_BYTES + b_shift * item, 0xA5, dtype=np.uint8).view(t)
+    dB = to_device(np.concatenate([guard, wl.nan_buffer(w["dtype"], n), guard]))
     p = wl.Permutation(handle, w)
-    pa, pb = dA.data_ptr() + a_shift * item, dB.data_ptr() + b_shift * item
+    pa, pb = dA.data_ptr() + a_shift * item, dB.data_ptr() + front * item
     info = p.info(pa, pb)
     st = p.run(pa, pb, torch.cuda.current_stream().cuda_stream)
     torch.cuda.synchronize()
     p.close()
     api.check(st, "hiptensorPermutation " + w["name"])
-    out = dB.cpu().numpy().view(t)[b_shift:]
+    out = dB.cpu().numpy().view(t)
+    for side in (out[:front], out[front + n:]):
+        assert np.all(side.view(np.uint8) == 0xA5), f"{w['name']}: stored beyond B ({info['kernel_name']})"
+    out = out[front:front + n]
     return (out, info) if return_info else out

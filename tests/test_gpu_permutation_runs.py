@@ -1,6 +1,6 @@
 """GPU parity of the linear permutation (a shared fastest mode, B written in 16-byte vectors): runs of exactly a vector, of a vector
-and a few elements more, long odd ones; vectors that span two runs at the front and at the end of A, where only part of
-them may be loaded; element counts that are no multiple of the vector; bases off their alignment; both forms of the element operation."""
+and a few elements more, long odd ones; vectors that span two runs, at the front and at the end of A among them; element counts that are no multiple of
+the vector; bases off their alignment; both forms of the element operation."""
 import pytest
 
 import gpu_util

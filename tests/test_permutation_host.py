@@ -3,11 +3,12 @@ reference's order (library/src/permutation/hiptensor_permutation.cpp:77-155, 173
 fusion and kernel choice of the planner."""
 import ctypes as C
 import os
+import subprocess
 
 import pytest
 
 import perm_cases
-from hiptensor_amd import api
+from hiptensor_amd import _lib, api
 from hiptensor_amd import workloads as wl
 
 
@@ -212,3 +213,15 @@ def test_every_validation_case_plans(host_handle):
             i = p.info()
             p.close()
             assert i["kernel_name"], w["name"]
+
+
+def test_vectors_at_any_element_stay_inside(tmp_path):
+    """tests/cpp/perm_bounds.cpp: every load and store of the kernels that move 16-byte vectors at any element, walked on
+    the host with the planner's own choices and the kernels' own address functions (kernels/perm_addr.hpp)."""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    src, out = os.path.join(root, "tests", "cpp", "perm_bounds.cpp"), tmp_path / "perm_bounds"
+    subprocess.run(["g++", "-std=c++17", "-O1", "-I" + os.path.join(root, "include"), src, "-o", str(out),
+                    "-L" + os.path.dirname(_lib.LIB_PATH), "-lhiptensor_amd", "-Wl,-rpath," + os.path.dirname(_lib.LIB_PATH)],
+                   check=True, capture_output=True)
+    r = subprocess.run([str(out)], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0 and r.stdout.strip().splitlines()[-1] == "ok", (r.stdout[-2000:], r.stderr)
