@@ -3,7 +3,7 @@
 // Argument checks, their order, status codes and messages follow the reference,
 // library/src/permutation/hiptensor_permutation.cpp:44-279.  Below the checks the reference
 // walks a registry of Composable Kernel element-wise instances until one accepts the problem;
-// here the problem is fused and mapped to one of four memory-bound kernels
+// here the problem is fused and mapped to one of eight memory-bound kernels
 // (permute_plan.cpp) and launched once on the caller's stream.
 #include <cmath>
 #include <cstdio>

@@ -695,8 +695,8 @@ namespace hiptk
         // wastes the lanes that overhang them, and needs vectors that divide the run; here a vector is any V consecutive
         // elements of B, taken from A in one load at whatever address they have there (global memory takes 16-byte loads
         // and stores at any multiple of the element), or in two where the vector spans the end of a run.
-        // f32 21.79.79.20.8.7 -> (0,1,3,4,5,2), 587 MB: 443 us in tiles, 203 here (5.8 TB/s); f32 30.7.61.7.7.65 ->
-        // (0,4,2,3,1,5), 163 MB in runs of 120 bytes: 468 -> 91 us (3.6 TB/s: the run's ends share lines with others').
+        // f32 21.79.79.20.8.7 -> (0,1,3,4,5,2), 587 MB: 447 us in tiles, 198 here (5.9 TB/s); f32 30.7.61.7.7.65 ->
+        // (0,4,2,3,1,5), 163 MB in runs of 120 bytes: 470 -> 81 us (4.0 TB/s: the run's ends share lines with others').
         // A thread moves U vectors, both loads of each in flight with the others'.
         template <typename T, int U>
         __global__ __launch_bounds__(PERM_THREADS) void permute_runs_kernel(RArgs a)
