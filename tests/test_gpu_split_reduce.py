@@ -59,14 +59,14 @@ def test_reduction_forms(gpu_handle, oracle_mod, dtype, m, n):
 K_TILE = {"f16": 64, "bf16": 64, "f32": 16, "f64": 16, "c32": 8, "c64": 8}
 
 
-def _one(handle, oracle_mod, dtype, m, n, k_tiles, split, beta, table=False, alias=False):
-    k = k_tiles * K_TILE[dtype]
+def _one(handle, oracle_mod, dtype, m, n, k_tiles, split, beta, table=False, alias=False, compute=None):
+    k = k_tiles * (64 if compute == api.HIPTENSOR_COMPUTE_16F else K_TILE[dtype])
     a = 1.1 + 0.4j if dtype.startswith("c") else 1.5
     b = None if not beta else 0.6 - 0.3j if dtype.startswith("c") else 0.75
     modes = list(range(len(m))), list(range(10, 10 + len(n)))
     ext = {**dict(zip(modes[0], m)), **dict(zip(modes[1], n)), 20: k}
     d = modes[0] + modes[1]
-    w = wl.make_workload(dtype, cases.COMPUTE[dtype], modes[0] + [20], modes[1] + [20], d[::-1] if table else d, ext, a, b,
+    w = wl.make_workload(dtype, compute or cases.COMPUTE[dtype], modes[0] + [20], modes[1] + [20], d[::-1] if table else d, ext, a, b,
                          name=f"reduce_{dtype}_{'x'.join(map(str, m))}_{'x'.join(map(str, n))}_{k}")
     inp = wl.host_inputs(w)
     exp = cases.logical_view(w, oracle_mod.contract(w, inp["A"], inp["B"], inp["C"]))
@@ -95,3 +95,10 @@ def test_large_outputs(gpu_handle, oracle_mod, dtype, m, n):
     last whole vector; D apart from C and in its place, computed offsets and ones from tables (rows along D and across it)."""
     for beta, table, alias in ((False, False, False), (True, False, True), (True, True, True)):
         _one(gpu_handle, oracle_mod, dtype, m, n, 22, 16, beta, table, alias)
+
+
+@pytest.mark.parametrize("dtype,compute", [("f64", api.HIPTENSOR_COMPUTE_32F), ("f32", api.HIPTENSOR_COMPUTE_16F)])
+def test_large_outputs_computed_narrower(gpu_handle, oracle_mod, dtype, compute):
+    """The partials' type is not the tensors' (f64 data: four f32 sums make 32 bytes of D)."""
+    for m, n, alias in (((725,), (725,), False), ((29, 25), (726,), True)):
+        _one(gpu_handle, oracle_mod, dtype, m, n, 22, 16, alias, False, alias, compute)
