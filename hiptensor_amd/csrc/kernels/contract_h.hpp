@@ -430,7 +430,7 @@ namespace hiptk
     // DEEP: two slabs of C in flight also for the 128-wide wave tiles (for kernels whose main loop
     // leaves the registers for it).
     template <typename Tr, int WP, int WQ, int TP, int TQ, int LDSCAP, bool DEEP, typename Acc>
-    __device__ __forceinline__ void epilogue_acc(const KArgs& a, const Acc acc, uint16_t* lds, int p0, int q0, int p_own, int q_own)
+    __device__ __forceinline__ void epilogue_acc(const KArgs& a, const Acc acc, uint16_t* lds, int p0, int q0, int p_own, int q_own, int slice)
     {
         constexpr int QUADS = Acc::QUADS;
         constexpr int WTP = TP * 32, WTQ = TQ * 32;
@@ -448,7 +448,7 @@ namespace hiptk
         const float beta  = (float)a.beta[0];
         if(a.split_k > 1)
         {
-            float* ws = (float*)a.ws + (size_t)blockIdx.z * (size_t)a.P * (size_t)a.Q;
+            float* ws = (float*)a.ws + (size_t)slice * (size_t)a.P * (size_t)a.Q;
 #pragma unroll
             for(int u = 0; u < QUADS; u++)
             {
@@ -968,15 +968,15 @@ namespace hiptk
 
     // ... for accumulators of v_mfma_f32_32x32x16 blocks
     template <typename Tr, int WP, int WQ, int TP, int TQ, int LDSCAP, bool DEEP = false>
-    __device__ __forceinline__ void epilogue_h(const KArgs& a, f32x16_t (&acc)[TP][TQ], uint16_t* lds, int p0, int q0, int p_own, int q_own)
+    __device__ __forceinline__ void epilogue_h(const KArgs& a, f32x16_t (&acc)[TP][TQ], uint16_t* lds, int p0, int q0, int p_own, int q_own, int slice)
     {
-        epilogue_acc<Tr, WP, WQ, TP, TQ, LDSCAP, DEEP>(a, Acc32<TP, TQ>{acc}, lds, p0, q0, p_own, q_own);
+        epilogue_acc<Tr, WP, WQ, TP, TQ, LDSCAP, DEEP>(a, Acc32<TP, TQ>{acc}, lds, p0, q0, p_own, q_own, slice);
     }
     // ... and of v_mfma_f32_16x16x32 blocks (TP x TQ still counts blocks of 32 x 32)
     template <typename Tr, int WP, int WQ, int TP, int TQ, int LDSCAP, bool DEEP = false>
-    __device__ __forceinline__ void epilogue_h16(const KArgs& a, f32x4_t (&acc)[2 * TP][2 * TQ], uint16_t* lds, int p0, int q0, int p_own, int q_own)
+    __device__ __forceinline__ void epilogue_h16(const KArgs& a, f32x4_t (&acc)[2 * TP][2 * TQ], uint16_t* lds, int p0, int q0, int p_own, int q_own, int slice)
     {
-        epilogue_acc<Tr, WP, WQ, TP, TQ, LDSCAP, DEEP>(a, Acc16<TP, TQ>{acc}, lds, p0, q0, p_own, q_own);
+        epilogue_acc<Tr, WP, WQ, TP, TQ, LDSCAP, DEEP>(a, Acc16<TP, TQ>{acc}, lds, p0, q0, p_own, q_own, slice);
     }
 
     template <typename Tr,
@@ -1009,15 +1009,15 @@ namespace hiptk
         const int wp   = wave / WQ;
         const int wq   = wave % WQ;
 
-        int tp, tq;
-        tile_coords(blockIdx.x, a.tiles_p, a.tiles_q, tp, tq);
+        int tp, tq, slice;
+        tile_coords(a, tp, tq, slice);
         // rows / columns from p_own / q_own on are this tile's to store; with shift_p / shift_q the
         // last tile is moved back to end exactly at P / Q (and recomputes some of its neighbour's)
         const int p_own = tp * BP, q_own = tq * BQ;
         const int p0    = (a.shift_p && p_own + BP > a.P) ? a.P - BP : p_own;
         const int q0    = (a.shift_q && q_own + BQ > a.Q) ? a.Q - BQ : q_own;
 
-        const int kt_begin = blockIdx.z * a.ktiles_per_split;
+        const int kt_begin = slice * a.ktiles_per_split;
         int       kt_end   = kt_begin + a.ktiles_per_split;
         const int kt_all   = (a.K + BK - 1) / BK;
         if(kt_end > kt_all)
@@ -1243,7 +1243,7 @@ namespace hiptk
             buf ^= 1;
         }
 
-        epilogue_h<Tr, WP, WQ, TP, TQ, 2 * STAGE * 2>(a, acc, lds, p0, q0, p_own, q_own);
+        epilogue_h<Tr, WP, WQ, TP, TQ, 2 * STAGE * 2>(a, acc, lds, p0, q0, p_own, q_own, slice);
     }
 
     template <typename Tr,

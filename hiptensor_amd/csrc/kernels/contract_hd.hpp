@@ -192,14 +192,14 @@ namespace hiptk
         const int wp   = wave / WQ;
         const int wq   = wave % WQ;
 
-        int tp, tq;
-        tile_coords(blockIdx.x, a.tiles_p, a.tiles_q, tp, tq);
+        int tp, tq, slice;
+        tile_coords(a, tp, tq, slice);
         const int p_own = tp * BP, q_own = tq * BQ;
         const int p0    = (a.shift_p && p_own + BP > a.P) ? a.P - BP : p_own;
         const int q0    = (a.shift_q && q_own + BQ > a.Q) ? a.Q - BQ : q_own;
 
         // This slice's K tiles: nt whole ones, and the 16-element tail when the slice ends at K
-        const int     kt_begin = blockIdx.z * a.ktiles_per_split;
+        const int     kt_begin = slice * a.ktiles_per_split;
         const HdSlice sl       = hd_slice(a.K, kt_begin, a.ktiles_per_split);
         const int     nt = sl.nt, n_load = sl.n_load, kmax = sl.kmax, k00 = sl.k00, klast = sl.klast;
         const bool    half = sl.half != 0;
@@ -523,7 +523,7 @@ namespace hiptk
 #pragma unroll
             for(int j = 0; j < TQ; j++)
                 asm volatile("" : "+a"(acc[i][j]));
-        epilogue_h<Tr, WP, WQ, TP, TQ, G::EPI, true>(a, acc, lds, p0, q0, p_own, q_own);
+        epilogue_h<Tr, WP, WQ, TP, TQ, G::EPI, true>(a, acc, lds, p0, q0, p_own, q_own, slice);
         // the loads beyond the K range (into the spare KiB, and of table entries) must not outlive
         // the workgroup's LDS
         __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));

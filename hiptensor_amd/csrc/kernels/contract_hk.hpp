@@ -219,13 +219,13 @@ namespace hiptk
         const int wp   = wave / WQ;
         const int wq   = wave % WQ;
 
-        int tp, tq;
-        tile_coords(blockIdx.x, a.tiles_p, a.tiles_q, tp, tq);
+        int tp, tq, slice;
+        tile_coords(a, tp, tq, slice);
         const int p_own = tp * BP, q_own = tq * BQ;
         const int p0    = (a.shift_p && p_own + BP > a.P) ? a.P - BP : p_own;
         const int q0    = (a.shift_q && q_own + BQ > a.Q) ? a.Q - BQ : q_own;
 
-        const int     kt_begin = blockIdx.z * a.ktiles_per_split;
+        const int     kt_begin = slice * a.ktiles_per_split;
         const HkSlice sl       = hk_slice(a.K, kt_begin, a.ktiles_per_split);
         const int     nt = sl.nt, klast = sl.klast, tail = sl.tail;
 
@@ -528,7 +528,7 @@ namespace hiptk
 #pragma unroll
             for(int j = 0; j < NBQ; j++)
                 asm volatile("" : "+a"(acc[i][j]));
-        epilogue_h16<Tr, WP, WQ, TP, TQ, G::LDS_BYTES, true>(a, acc, lds, p0, q0, p_own, q_own);
+        epilogue_h16<Tr, WP, WQ, TP, TQ, G::LDS_BYTES, true>(a, acc, lds, p0, q0, p_own, q_own, slice);
     }
 
     template <typename Tr, bool XKF, bool YKF, int BQ, int NSX, int NSY, int SP>

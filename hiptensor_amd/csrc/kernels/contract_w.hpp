@@ -427,7 +427,7 @@ namespace hiptk
     // lane's column in it; rows / columns from p_own / q_own on are the workgroup tile's to store.
     template <typename Tr, int TP, int TQ>
     __device__ __forceinline__ void
-        epilogue_w(const KArgs& a, typename Tr::Acc (&acc)[TP][TQ], int pw, int qw, int p_own, int q_own, int lane)
+        epilogue_w(const KArgs& a, typename Tr::Acc (&acc)[TP][TQ], int pw, int qw, int p_own, int q_own, int slice, int lane)
     {
         typedef typename Tr::E E;
         typedef typename Tr::O O;
@@ -436,7 +436,7 @@ namespace hiptk
         auto                   q_in = [&](int q) { return q >= q_own && q < a.Q; };
         if(a.split_k > 1)
         {
-            O* ws = (O*)a.ws + (size_t)blockIdx.z * (size_t)a.P * (size_t)a.Q;
+            O* ws = (O*)a.ws + (size_t)slice * (size_t)a.P * (size_t)a.Q;
 #pragma unroll
             for(int i = 0; i < TP; i++)
 #pragma unroll
@@ -545,8 +545,8 @@ namespace hiptk
         const int wp   = wave / WQ;
         const int wq   = wave % WQ;
 
-        int tp, tq;
-        tile_coords(blockIdx.x, a.tiles_p, a.tiles_q, tp, tq);
+        int tp, tq, slice;
+        tile_coords(a, tp, tq, slice);
         // rows / columns from p_own / q_own on are this tile's to store; with shift_p / shift_q the
         // last tile is moved back to end exactly at P / Q (and recomputes some of its neighbour's)
         const int p_own = tp * BP, q_own = tq * BQ;
@@ -555,7 +555,7 @@ namespace hiptk
         auto      p_in  = [&](int p) { return p >= p_own && p < a.P; };
         auto      q_in  = [&](int q) { return q >= q_own && q < a.Q; };
 
-        const int kt_begin = blockIdx.z * a.ktiles_per_split;
+        const int kt_begin = slice * a.ktiles_per_split;
         int       kt_end   = kt_begin + a.ktiles_per_split;
         const int kt_all   = (a.K + BK - 1) / BK;
         if(kt_end > kt_all)
@@ -687,7 +687,7 @@ namespace hiptk
             buf ^= 1;
         }
 
-        epilogue_w<Tr, TP, TQ>(a, acc, p0 + wp * WTP, q0 + wq * WTQ + Tr::q_of(lane), p_own, q_own, lane);
+        epilogue_w<Tr, TP, TQ>(a, acc, p0 + wp * WTP, q0 + wq * WTQ + Tr::q_of(lane), p_own, q_own, slice, lane);
     }
 
     template <typename Tr, int BP, int BQ, int BK>

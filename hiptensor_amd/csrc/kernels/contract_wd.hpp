@@ -230,13 +230,13 @@ namespace hiptk
         const int wq   = WK ? 0 : wave & 1;
         constexpr int ROWS = G::ROWS;
 
-        int tp, tq;
-        tile_coords(blockIdx.x, a.tiles_p, a.tiles_q, tp, tq);
+        int tp, tq, slice;
+        tile_coords(a, tp, tq, slice);
         // (no tile is moved back; a tile that overhangs P or Q reads the padding of the row tables, offset 0,
         // and stores nothing there)
         const int p0 = tp * G::BP, q0 = tq * G::BQ;
 
-        int       kt_begin = blockIdx.z * a.ktiles_per_split;
+        int       kt_begin = slice * a.ktiles_per_split;
         int       kt_end   = kt_begin + a.ktiles_per_split;
         const int kt_all   = (a.K + BK - 1) / BK; // the last tile may hold fewer than BK k
         if(kt_end > kt_all)
@@ -521,14 +521,14 @@ namespace hiptk
             if(whole_k)
                 epi.store(a, acc);
             else
-                epilogue_w<Tr, TP, TQ>(a, acc, p0, q0 + Tr::q_of(lane), p0, q0, lane);
+                epilogue_w<Tr, TP, TQ>(a, acc, p0, q0 + Tr::q_of(lane), p0, q0, slice, lane);
         }
         else
         {
             if(whole_k)
                 epi.store(a, acc);
             else
-                epilogue_w<Tr, TP, TQ>(a, acc, p0 + wp * 32, q0 + wq * 32 + Tr::q_of(lane), p0, q0, lane);
+                epilogue_w<Tr, TP, TQ>(a, acc, p0 + wp * 32, q0 + wq * 32 + Tr::q_of(lane), p0, q0, slice, lane);
             // the loads beyond the K range (into the spare KiB) must not outlive the workgroup's LDS
             __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
         }

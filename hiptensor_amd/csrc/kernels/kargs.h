@@ -21,6 +21,7 @@ namespace hiptk
         int32_t split_k;
         int32_t bilinear;
         int32_t tiles_p, tiles_q;
+        int32_t slice_bands; // 1: the XCDs share out slices, not the tiles of each slice (tile_coords)
         int32_t xk_stride, yk_stride; // element stride of k when the K modes fused into one
         int32_t cd_affine; // 1: C / D offsets are p * stride + q * stride, no table lookups
         int32_t dp_stride, dq_stride, cp_stride, cq_stride;
@@ -86,26 +87,36 @@ namespace hiptk
     const KernelEntry* entries_f32_as_f16(int* count);
     const KernelEntry* entries_f32_as_bf16(int* count);
 
-    // XCD-aware mapping of the linear workgroup id to an output tile.  Workgroups are
+    // XCD-aware mapping of the workgroup id to a K slice and an output tile.  Workgroups are
     // handed to the 8 XCDs round-robin, so ids that are congruent mod 8 share an L2.
     // Give each XCD a contiguous band of the tile space and walk that band in
     // column-groups of GROUP rows so that the X rows / Y columns a band touches
-    // stay resident in that XCD's L2.
-    __device__ inline void tile_coords(int wg, int tiles_p, int tiles_q, int& tp, int& tq)
+    // stay resident in that XCD's L2.  With `slice_bands` the bands run through all slices'
+    // tiles, slice after slice, so that the tiles of a slice, which read the same panels, meet
+    // in one or two L2s instead of all eight.
+    __device__ inline void tile_coords(const KArgs& a, int& tp, int& tq, int& slice)
     {
         // XCD x runs the workgroups wg = x, x + 8, ...: base = total / 8 of them, one more for the
-        // first total % 8 XCDs; give it the contiguous range of tiles that starts after its
+        // first total % 8 XCDs; give it the contiguous range of work that starts after its
         // predecessors' shares
-        const int total = tiles_p * tiles_q;
-        const int xcd = wg & 7, nth = wg >> 3;
-        const int base = total >> 3, rem = total & 7;
-        const int lin  = xcd * base + (xcd < rem ? xcd : rem) + nth;
+        const uint32_t tiles = (uint32_t)a.tiles_p * (uint32_t)a.tiles_q;
+        const uint32_t total = a.slice_bands ? tiles * (uint32_t)a.split_k : tiles;
+        const uint32_t wg    = a.slice_bands ? blockIdx.x + tiles * blockIdx.z : blockIdx.x;
+        const uint32_t xcd = wg & 7, nth = wg >> 3;
+        const uint32_t base = total >> 3, rem = total & 7;
+        uint32_t       lin  = xcd * base + (xcd < rem ? xcd : rem) + nth;
+        slice               = (int)blockIdx.z;
+        if(a.slice_bands)
+        {
+            slice = (int)(lin / tiles);
+            lin -= (uint32_t)slice * tiles;
+        }
         constexpr int GROUP = 4;
-        const int     band  = GROUP * tiles_q;
-        const int     g     = lin / band;
+        const int     band  = GROUP * a.tiles_q;
+        const int     g     = (int)lin / band;
         const int     first = g * GROUP;
-        const int     rows  = (tiles_p - first) < GROUP ? (tiles_p - first) : GROUP;
-        const int     r     = lin - g * band;
+        const int     rows  = (a.tiles_p - first) < GROUP ? (a.tiles_p - first) : GROUP;
+        const int     r     = (int)lin - g * band;
         tp                  = first + r % rows;
         tq                  = r / rows;
     }

@@ -102,3 +102,12 @@ def test_large_outputs_computed_narrower(gpu_handle, oracle_mod, dtype, compute)
     """The partials' type is not the tensors' (f64 data: four f32 sums make 32 bytes of D)."""
     for m, n, alias in (((725,), (725,), False), ((29, 25), (726,), True)):
         _one(gpu_handle, oracle_mod, dtype, m, n, 22, 16, alias, False, alias, compute)
+
+
+@pytest.mark.parametrize("dtype", list(TILES))
+@pytest.mark.parametrize("m,n", [((1,), (3,)), ((70,), (130,)), ((200,), (14, 10))])
+def test_slices_shared_out_between_dies(gpu_handle, oracle_mod, dtype, m, n):
+    """Two hundred K tiles in 29 and 50 slices of 1 to 12 (35 for complex f64) output tiles: workgroups are then dealt to
+    the dies slice by slice, in shares that do not end where a slice does."""
+    for split in (32, 64):
+        _one(gpu_handle, oracle_mod, dtype, m, n, 200, split, split == 32)
