@@ -524,25 +524,38 @@ namespace hipta
 
         v.x_max_off = mxp + mxk;
         v.y_max_off = myq + myk;
-        // 16-byte vectors that start on 16-byte multiples of the tensor's base
+        // what the starts of all 16-byte vectors are multiples of, from the tensor's base: 16 bytes, else 4, else nothing.
+        // (A vector starts at a multiple of its length along the dim it runs along, so it is a question of the other strides.)
         {
             const int want = v.elem_bytes >= 1 && v.elem_bytes <= 16 ? 16 / v.elem_bytes : 0;
-            auto aligned = [want](const std::vector<int32_t>& rows, int64_t nrows, const std::vector<int32_t>& ks, int64_t nk,
-                                  bool kfast, int vec, bool shifted) {
-                if(want == 0 || vec != want || (!kfast && shifted))
-                    return false;
-                for(int64_t r = 0; r < nrows; r += kfast ? 1 : vec)
-                    if(rows[(size_t)r] % vec != 0)
-                        return false;
-                for(int64_t k = 0; k < nk; k += kfast ? vec : 1)
-                    if(ks[(size_t)k] % vec != 0)
+            auto strides_multiple = [](const std::vector<Dim>& d, size_t from, int64_t Dim::*stride, int64_t unit) {
+                for(size_t i = from; i < d.size(); i++)
+                    if(d[i].*stride % unit != 0)
                         return false;
                 return true;
             };
-            v.xy_aligned = (aligned(v.xp, v.P, v.xk, v.K, v.x_kfast != 0, v.x_vec, v.shift_p != 0)
-                            && aligned(v.yq, v.Q, v.yk, v.K, v.y_kfast != 0, v.y_vec, v.shift_q != 0))
-                               ? 1
-                               : 0;
+            auto aligned = [&](const std::vector<Dim>& rows, int64_t nrows, int64_t Dim::*stride, bool kfast, int vec, bool shifted, int64_t unit) {
+                if(want == 0 || vec != want)
+                    return false;
+                // (a tile that is moved back ends at the last row: its vectors start a multiple of 32 rows before it)
+                if(!kfast && shifted && (unit >= want || nrows % unit != 0))
+                    return false;
+                return strides_multiple(rows, kfast || vec == 1 ? 0 : 1, stride, unit)
+                       && strides_multiple(v.kdims, kfast && vec > 1 ? 1 : 0, stride, unit);
+            };
+            v.xy_aligned = 0;
+            for(int bytes : {4, 16})
+            {
+                const int64_t unit = std::max(1, bytes / std::max(1, v.elem_bytes));
+                if(aligned(v.pdims, v.P, &Dim::sx, v.x_kfast != 0, v.x_vec, v.shift_p != 0, unit)
+                   && aligned(v.qdims, v.Q, &Dim::sy, v.y_kfast != 0, v.y_vec, v.shift_q != 0, unit))
+                    v.xy_aligned = bytes;
+            }
+            // do the runs of memory that a K tile reads (rows of a k-contiguous operand, else the rows at one k) start at
+            // 128-byte lines?
+            const int64_t line = std::max(1, 128 / std::max(1, v.elem_bytes));
+            v.x_lines          = strides_multiple(v.x_kfast ? v.pdims : v.kdims, 0, &Dim::sx, line) ? 1 : 0;
+            v.y_lines          = strides_multiple(v.y_kfast ? v.qdims : v.kdims, 0, &Dim::sy, line) ? 1 : 0;
         }
 
         // k-contiguous operand: which neighbour of a vector is its neighbour in memory too, the next row's or the next

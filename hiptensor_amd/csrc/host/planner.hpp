@@ -64,8 +64,10 @@ namespace hipta
         // vectors run along a row (column) index that is one contiguous run whose extent is not a
         // multiple of the vector: tiles that would overhang are moved back to end at P (Q)
         int shift_p = 0, shift_q = 0;
-        // every 16-byte vector of X and Y starts a multiple of 16 bytes from its tensor's base
+        // every 16-byte vector of X and Y starts a multiple of this many bytes from its tensor's base: 16, 4 or 0 (neither)
         int xy_aligned = 0;
+        // the runs of memory along X's / Y's vectors start at multiples of 128 bytes
+        int x_lines = 0, y_lines = 0;
         // largest element offset of X / Y that the tables address
         int64_t xp_stride = 0, yq_stride = 0; // with cd_affine: element stride of the one row mode of X / column mode of Y
         int64_t x_max_off = 0, y_max_off = 0;

@@ -180,7 +180,7 @@ namespace hipta
         double round_extra_us = 0.0;
         if(v.cls == HIPTK_F64 && s.bp * s.bq >= 16384 && !(v.x_kfast && v.y_kfast))
             r = TileRate{0.74, 0.74};
-        if(class_flops_per_clk_cu(v.cls) == 4096.0 && s.direct && s.bk == 64)
+        if(class_flops_per_clk_cu(v.cls) == 4096.0 && s.direct && s.bk == 64 && s.bp * s.bq >= 65536)
         {
             // The 256 x 256 tile on 16 x 16 x 32 MFMAs whose operand tiles are loaded straight into LDS in K tiles of
             // 64 (four waves).  4096^3 f16 scale, one device: both operands k-contiguous 98.5 us (main loop 84.2,
@@ -229,6 +229,23 @@ namespace hipta
             const double f = kper / s.bk < 24 ? 0.9 : v.bilinear ? 0.95 : (v.x_kfast || v.y_kfast) ? 0.96 : 1.005;
             r.alone *= f;
             r.full *= f;
+        }
+        // The 16-bit direct-load tiles of up to 128 rows: a K step of 64 takes a workgroup's share of the LDS (its loads written,
+        // its operands read), the same for one workgroup on a CU and for two; rows that do not start at 128-byte lines
+        // take half as long again to arrive.
+        const bool ring_step = class_flops_per_clk_cu(v.cls) == 4096.0 && s.direct && s.bp * s.bq < 49152;
+        double     step_us   = 0.0;
+        if(ring_step)
+        {
+            const bool small = s.bp * s.bq <= 4096, lines = v.x_lines && v.y_lines;
+            const int  kf    = (v.x_kfast ? 1 : 0) + (v.y_kfast ? 1 : 0);
+            step_us          = small ? (lines ? (kf == 2 ? 0.16 : kf == 1 ? 0.17 : 0.20) : (kf == 2 ? 0.245 : 0.235))
+                                     : (lines ? (kf == 2 ? 0.285 : kf == 1 ? 0.30 : 0.35) : (kf == 2 ? 0.41 : 0.375));
+            round_extra_us   = 1.6;
+            // (three and more of them on a CU: larger tiles win earlier than their estimates say, 4704 x 1204 x 3456 50.2 us on
+            // 256 x 128 and 62.1 on 64 x 64, 5472 x 1732 x 2688 63.5 on 256 x 256 and 77.4 on 128 x 64)
+            if(per_cu >= 3)
+                step_us *= 1.3;
         }
         if(s.direct && class_flops_per_clk_cu(v.cls) != 4096.0)
         {
@@ -282,16 +299,25 @@ namespace hipta
         const double frac     = sharing <= 1.0 ? r.alone : std::min(sharing * r.alone, r.full);
         const double flops_wg = class_flops_per_mac(v.cls) * (double)s.bp * s.bq * kper;
         const double cu_rate  = class_flops_per_clk_cu(v.cls) * dev.clock_ghz * 1e3; // flop / us
-        double       us       = per_cu * flops_wg / (frac * cu_rate);
+        double       us       = ring_step ? per_cu * kper / s.bk * step_us : per_cu * flops_wg / (frac * cu_rate);
         // memory floor: every operand once (+ C and D)
         const double bytes = ((double)v.P * v.K + (double)v.Q * v.K + (double)v.P * v.Q * (v.bilinear ? 2 : 1))
                              * v.elem_bytes;
-        us = std::max(us, bytes / (dev.hbm_gbs * 1e3 * 0.6));
+        // (the rings of the 16-bit tiles of up to 128 rows keep HBM busier, and the closer their steps come to it the more of
+        // both shows: 8192 x 16 x 8192 on 64 x 64 tiles in two slices 30.2 us, in one 41.5, in
+        // four 33.1)
+        if(ring_step)
+            us = std::cbrt(us * us * us + std::pow(bytes / (dev.hbm_gbs * 1e3 * 0.72), 3.0));
+        else
+            us = std::max(us, bytes / (dev.hbm_gbs * 1e3 * 0.6));
         // split-K slices of different tiles share nothing in time: every workgroup's operand panels come through
         // the fabric (256 x 256 x 65536 f16 in 32 slices: 16 tiles of 64 x 64 move 2.7e8 B for 6.7e7 algorithmic
         // and take 40.5 us, 4 tiles of 128 x 128 move half of that and take 33.4)
+        // (a little more of them where an XCD takes whole slices, whose tiles then meet in its L2: launch.hip; f64 110 x 324 x
+        // 112500 on 32 x 32 tiles in 16 slices 231 us, on 64 x 64 in 64 190)
+        const bool slice_bands = split >= 8 && std::ceil(ktiles / split) * split >= 160;
         if(split > 1)
-            us = std::max(us, tiles * (double)(s.bp + s.bq) * (double)v.K * v.elem_bytes / (dev.hbm_gbs * 1e3 * 1.4));
+            us = std::max(us, tiles * (double)(s.bp + s.bq) * (double)v.K * v.elem_bytes / (dev.hbm_gbs * 1e3 * (slice_bands ? 1.75 : 1.4)));
         // launch, and prologue + epilogue of every round of workgroups on a CU
         // (a workgroup's epilogue moves its output tile, and C, at about 30 GB/s per CU)
         const double tile_io = (double)s.bp * s.bq * v.elem_bytes * (v.bilinear ? 2.0 : 1.0) / 30e3;
@@ -309,7 +335,10 @@ namespace hipta
             // it lies in 64 12.1, packed and in 16 19.6).  Over 570 shapes the choice takes 1.03 of the time of the best
             // tile and split (1.06 with 0.25 a slice throughout).
             double per_slice = 0.25 * split;
-            if(split > 16)
+            // (the 16-bit rings start a slice's first loads all at once: 36 x 216 x 36540 bf16 20.6 / 13.2 / 9.9 / 9.5 us in 8 / 16 / 32 / 64)
+            if(ring_step)
+                per_slice = 0.03 * split + 0.25 * std::max(0.0, 4.0 - kper / s.bk);
+            else if(split > 16)
                 per_slice = std::min(per_slice, 4.0 + 0.05 * (split - 16) + 0.2 * std::max(0.0, 16.0 - kper / s.bk));
             us += 2.0 * ws / bw + 3.0 + per_slice;
         }

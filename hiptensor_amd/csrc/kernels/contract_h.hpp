@@ -141,6 +141,16 @@ namespace hiptk
         }
     };
 
+    // v_mfma_f32_16x16x32 as the compiler knows it (contract_hk.hpp's K tail, contract_hm.hpp)
+    __device__ inline f32x4_t hk_mfma16(TraitsF16, u32x4_t x, u32x4_t y, f32x4_t acc)
+    {
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, x), __builtin_bit_cast(half8_t, y), acc, 0, 0, 0);
+    }
+    __device__ inline f32x4_t hk_mfma16(TraitsBF16, u32x4_t x, u32x4_t y, f32x4_t acc)
+    {
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, x), __builtin_bit_cast(bf16x8_t, y), acc, 0, 0, 0);
+    }
+
     // LDS tile geometry of one operand (16-bit elements).
     template <bool KF, int BR, int BK>
     struct TileLds

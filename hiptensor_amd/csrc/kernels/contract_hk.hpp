@@ -184,16 +184,6 @@ namespace hiptk
     {
         asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
     }
-    // ... and the same MFMA as the compiler knows it, for the K tail
-    __device__ inline f32x4_t hk_mfma16(TraitsF16, u32x4_t x, u32x4_t y, f32x4_t acc)
-    {
-        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, x), __builtin_bit_cast(half8_t, y), acc, 0, 0, 0);
-    }
-    __device__ inline f32x4_t hk_mfma16(TraitsBF16, u32x4_t x, u32x4_t y, f32x4_t acc)
-    {
-        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, x), __builtin_bit_cast(bf16x8_t, y), acc, 0, 0, 0);
-    }
-
     template <typename Tr, bool XKF, bool YKF, int BQ, int NSX, int NSY, int SP>
     __global__ void __launch_bounds__(256, 1) contract_hk_kernel(const KArgs a)
     {

@@ -192,6 +192,59 @@ namespace hiptk
         return (((row >> 3) ^ (2 * (k & 3))) << 3) | (row & 7);
     }
 
+    // ---- 16-bit kernel for tiles smaller than 256 (contract_hm.hpp): K tiles of 64, stages as above ----
+    // The K tiles one workgroup reduces, in the order it takes them: when the slice ends at K and K is not a
+    // multiple of 64, the tile with the last tail_k k comes first (its loads are the ones that need tests and may be
+    // more than a whole tile's, which the waits for any later tile then need not count), then the whole tiles.
+    struct HmSlice
+    {
+        int nt, tail_k, k00;
+    };
+    HIPTK_HD_FN HmSlice hm_slice(int K, int kt_begin, int ktiles_per_split)
+    {
+        HmSlice   s;
+        const int kt_all = (K + HK_BK - 1) / HK_BK;
+        const int kt_end = kt_begin + ktiles_per_split < kt_all ? kt_begin + ktiles_per_split : kt_all;
+        s.nt             = kt_end - kt_begin;
+        s.tail_k         = kt_end == kt_all ? K % HK_BK : 0;
+        s.k00            = kt_begin * HK_BK;
+        return s;
+    }
+    // k origin of the u-th tile taken
+    HIPTK_HD_FN int hm_origin(const HmSlice& s, int u)
+    {
+        return s.tail_k == 0 ? s.k00 + u * HK_BK : u == 0 ? s.k00 + (s.nt - 1) * HK_BK : s.k00 + (u - 1) * HK_BK;
+    }
+    // chunks of 8 rows are exchanged within a k-row so that the four k-rows a transposing read of 16 lanes touches lie
+    // in different banks; 32 rows are 64 bytes, four of which are in different banks as they are
+    template <int BR>
+    HIPTK_HD_FN int hm_row_pos(int row, int k)
+    {
+        return BR >= 64 ? hd_row_pos(row, k) : row;
+    }
+    // what the 16-byte slot s of a stage holds
+    template <bool KF, int BR>
+    HIPTK_HD_FN HdSlot hm_slot(int s)
+    {
+        if(KF)
+            return hk_slot<BR>(s);
+        HdSlot        o;
+        constexpr int cpr = BR / 8;
+        o.k               = s / cpr;
+        o.row             = hm_row_pos<BR>(8 * (s % cpr), o.k);
+        return o;
+    }
+    // The k (from the tile's origin, so -6 .. 63) that is loaded at k-position k of the tile of which only tail_k k lie
+    // inside K, or HM_ZERO for zeros.  With `chunks` (an operand is contiguous along k) the eight positions that K ends in
+    // hold the last eight k, for both operands alike.
+    constexpr int HM_ZERO = -64;
+    HIPTK_HD_FN int hm_tail_k(int k, int tail_k, bool chunks)
+    {
+        if(chunks && (k | 7) >= tail_k && (k & ~7) < tail_k)
+            return tail_k - 8 + (k & 7);
+        return k < tail_k ? k : HM_ZERO;
+    }
+
     template <bool KF, int BR>
     HIPTK_HD_FN HdSlot hd_slot(int s)
     {

@@ -52,6 +52,7 @@ namespace hiptk
         launch_fn   launch;
         int32_t     k_multiple; // 0: any K; else K must be a multiple of this and at least bk
         int32_t     mfma_k; // reduction depth of the MFMA instruction the tile is built on, where the selection tells tiles apart by it (else 0)
+        int32_t     vec_align; // k_multiple > 0: bytes that every 16-byte vector must start at a multiple of (0: 16)
     };
 
     // Each kernel translation unit contributes its table.
@@ -75,6 +76,8 @@ namespace hiptk
     const KernelEntry* entries_f16_hr192_rx(int* count);
     const KernelEntry* entries_bf16_hr192_kx(int* count);
     const KernelEntry* entries_bf16_hr192_rx(int* count);
+    const KernelEntry* entries_f16_hm(int* count);
+    const KernelEntry* entries_bf16_hm(int* count);
     const KernelEntry* entries_f16_v4(int* count);
     const KernelEntry* entries_f16_v2(int* count);
     const KernelEntry* entries_bf16_v4(int* count);

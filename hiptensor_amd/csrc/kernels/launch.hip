@@ -34,6 +34,8 @@ namespace hiptk
                                           entries_f16_hr192_rx,
                                           entries_bf16_hr192_kx,
                                           entries_bf16_hr192_rx,
+                                          entries_f16_hm,
+                                          entries_bf16_hm,
                                           entries_f16_aff,
                                           entries_bf16_aff,
                                           entries_f16_vec,
@@ -347,6 +349,12 @@ namespace hiptk
             }
         }
 
+        // What the 16-byte vectors of a direct-load kernel must start at multiples of, bytes
+        int vec_align(const KernelEntry& e)
+        {
+            return e.vec_align ? e.vec_align : 16;
+        }
+
         // The affine-K variant is preferred when the problem allows it; the table variant
         // serves every problem.
         const KernelEntry* find_entry(const hiptk_problem_t* p)
@@ -360,8 +368,8 @@ namespace hiptk
                     // a tile can only be moved back to end at P / Q if it fits into P / Q
                     if((p->shift_p && p->P < e.bp) || (p->shift_q && p->Q < e.bq))
                         continue;
-                    // the direct-load kernels: a restricted K tail, vectors on 16-byte multiples
-                    if(e.k_multiple > 0 && (p->K % e.k_multiple != 0 || p->K < e.bk || !p->xy_aligned))
+                    // the direct-load kernels: a restricted K tail, vectors on multiples of 16 (or 4) bytes
+                    if(e.k_multiple > 0 && (p->K % e.k_multiple != 0 || p->K < e.bk || p->xy_aligned < vec_align(e)))
                         continue;
                     // ... and they address an operand with 32-bit byte offsets
                     if(e.k_multiple > 0)
@@ -382,7 +390,7 @@ namespace hiptk
         }
 
         // The largest register-staged tile of the problem's class and layout: what runs in place of
-        // a direct-load kernel when an operand's base address is not 16-byte aligned.
+        // a direct-load kernel when an operand's base address is not aligned for it.
         const KernelEntry* staged_entry(const hiptk_problem_t* p)
         {
             const KernelEntry* best = nullptr;
@@ -410,7 +418,7 @@ namespace hiptk
                                   && e->y_kfast == (p->y_kfast != 0) && e->x_vec == p->x_vec && e->y_vec == p->y_vec;
             if(!resolved)
                 e = find_entry(p);
-            if(e && e->k_multiple > 0 && ((((uintptr_t)X) | ((uintptr_t)Y)) & 15) != 0)
+            if(e && e->k_multiple > 0 && ((((uintptr_t)X) | ((uintptr_t)Y)) & (uintptr_t)(vec_align(*e) - 1)) != 0)
                 e = resolved ? (const KernelEntry*)p->kernel_unaligned : staged_entry(p);
             return e;
         }

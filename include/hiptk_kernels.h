@@ -63,7 +63,7 @@ typedef struct hiptk_tile_info
     char    name[64];
     int32_t k_multiple; /* 0: operand tiles staged through registers, any K.  Otherwise the tile loads
                            them straight into LDS: K must be a multiple of this (1: any) and at least bk,
-                           and the problem xy_aligned                          */
+                           and the problem xy_aligned as far as the tile asks    */
     int32_t mfma_k;     /* 32: a 16-bit tile built on v_mfma_f32_16x16x32 (else 0)   */
 } hiptk_tile_info_t;
 
@@ -102,12 +102,12 @@ typedef struct hiptk_problem
                         its neighbour's rows and stores only its own).  Needs P >= the tile's rows;
                         tiles that do not fit are reported as unavailable                          */
     int32_t shift_q; /* likewise for the columns                                                    */
-    int32_t xy_aligned; /* 1: every 16-byte vector of X and Y starts a multiple of 16 bytes from its
-                           tensor's base (table entries at vector starts are multiples of the vector,
-                           no tile is moved back along a vector direction).  The kernels that load
-                           their operand tiles straight into LDS take only such problems, and only
-                           when the base addresses are 16-byte aligned too (checked at the launch,
-                           which otherwise runs the class's largest register-staged tile instead)  */
+    int32_t xy_aligned; /* 16 or 4: every 16-byte vector of X and Y starts a multiple of so many bytes from its
+                           tensor's base (table entries at vector starts are multiples of 16 or 4 bytes; 16 also says
+                           that no tile is moved back along a vector direction); else 0.  The kernels that load
+                           their operand tiles straight into LDS take only such problems (most of them only 16), and
+                           only when the base addresses are aligned likewise (checked at the launch, which
+                           otherwise runs the class's largest register-staged tile instead)  */
     int32_t x_max_off, y_max_off; /* largest element offset xp[p] + xk[k] (yq[q] + yk[k]) over p < P, k < K:
                                      the kernels that build load addresses from table entries they have
                                      themselves moved through LDS clamp every address to it, and the
@@ -121,7 +121,7 @@ typedef struct hiptk_problem
                                      neighbouring lanes load neighbouring memory.  Any value gives the same results */
     /* Filled by hiptk_resolve (zero otherwise): the registry entries this problem runs, looked up once
      * when the plan is made instead of at every launch.  `kernel` is what hiptk_kernel_name names;
-     * `kernel_unaligned` is what runs in its place when X or Y is not 16-byte aligned at the launch (the
+     * `kernel_unaligned` is what runs in its place when X or Y is not aligned for it at the launch (the
      * same entry, unless `kernel` loads operand tiles straight into LDS).  Both are tied to the fields
      * above: a caller that changes any of them afterwards clears these two (or resolves again). */
     const void *kernel, *kernel_unaligned;
