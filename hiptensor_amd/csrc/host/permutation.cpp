@@ -37,9 +37,9 @@ namespace
     }
 
     // HIPTENSOR_AMD_PERMUTE="kernel[,tile[,maxvec[,group]]]": kernel is auto | gather | tiled |
-    // rows | strip | grouped | runs (tiled and rows name the same preference: whichever of the two the
-    // layout admits; strip and grouped - which includes the shared-fastest-mode tiles - are
-    // taken wherever the layout admits them),
+    // rows | loose | strip | grouped | runs (tiled and rows name the same preference: whichever of the two the
+    // layout admits; loose is tiled with 16-byte vectors at any element; strip and grouped - which includes the
+    // shared-fastest-mode tiles - are taken wherever the layout admits them),
     // tile is 0..2 or -1, maxvec caps the vector width, group sets the band width of the
     // workgroup order.  For tests and experiments.
     hipta::PermuteTuning tuningFromEnv()
@@ -58,6 +58,8 @@ namespace
                 t.kernel = HIPTK_PERM_GATHER;
             else if(!std::strcmp(tok, "tiled") || !std::strcmp(tok, "rows"))
                 t.kernel = HIPTK_PERM_TILED;
+            else if(!std::strcmp(tok, "loose"))
+                t.kernel = HIPTK_PERM_TILED, t.loose = true;
             else if(!std::strcmp(tok, "strip"))
                 t.kernel = HIPTK_PERM_STRIP;
             else if(!std::strcmp(tok, "grouped"))

@@ -70,7 +70,7 @@ namespace hipta
         }
     }
 
-    PermuteStatus plan_permutation(const PermuteIn& in, const PermuteTuning& tune, hiptk_permute_t& out)
+    static PermuteStatus pick_kernel(const PermuteIn& in, const PermuteTuning& tune, hiptk_permute_t& out)
     {
         std::memset(&out, 0, sizeof(out));
         const size_t rank = in.lenA.size();
@@ -331,6 +331,14 @@ namespace hipta
             return PermuteStatus::OK;
         const int  full   = 16 / in.elem_bytes;
         const bool runs   = shared && ext[0] >= full && cap >= full; // a 16-byte vector spans two runs at the most
+        const int  sq    = (in.elem_bytes == 4 ? TILES4 : TILES2)[0].ti / 2;
+        const bool whole = ext[0] % sq == 0 && ext[jB] % sq == 0;
+        // strips of 32 rows and more of a tensor that a few hundred workgroups hold: smaller tiles spread it wider (f32
+        // 21311 x 57 8.1 us in strips, 4.7 in tiles of 64 x 64, f16 52296 x 56 7.7 and, grouped, 6.0; but
+        // f16 66.1684.35 -> (2,0,1), single elements on one side, 7.3 and 8.9)
+        const bool smallStrip = (stripJ || stripI) && tune.kernel < 0 && tune.tile < 0 && cap >= full && count <= (1 << 22)
+                                && std::min(ext[0], ext[jB]) >= 32 && std::max(ext[0], ext[jB]) >= 64
+                                && (in.elem_bytes == 4 || (ext[0] % 2 == 0 && ext[jB] % 2 == 0));
         if(tune.kernel == HIPTK_PERM_GATHER)
             kernel = HIPTK_PERM_GATHER;
         else if(tune.kernel == HIPTK_PERM_RUNS && runs)
@@ -341,16 +349,36 @@ namespace hipta
             kernel = shared ? HIPTK_PERM_ROWS : HIPTK_PERM_TILED;
         else if(count <= 16384)
             kernel = HIPTK_PERM_GATHER; // a launch's worth of latency either way
+        else if(!shared && count < (1 << 18) && !whole && tune.tile < 0 && tune.gather)
+            // Tiles make too few workgroups: f32 238 x 117 6.4 us in tiles, 2.3 here; f16 80 x 3213 8.1 and 3.1; f16
+            // 57 x 749 in strips 13.7 and 2.4.  (Extents that the small tiles cover to the last lane: 3.5-3.6 us in those.)
+            kernel = HIPTK_PERM_GATHER;
+        else if(smallStrip && in.elem_bytes == 4)
+            kernel = HIPTK_PERM_TILED;
+        else if(smallStrip && tryGrouped(true, false))
+            return PermuteStatus::OK;
         else if((stripJ && ext[0] >= 64) || (stripI && ext[jB] >= 64))
             kernel = HIPTK_PERM_STRIP;
         else if(shared && tune.tile < 0 && tryShared(false))
             return PermuteStatus::OK;
         else if(shared)
             kernel = ext[0] >= 16 ? HIPTK_PERM_ROWS : HIPTK_PERM_GATHER;
-        else if(tune.tile < 0 && tryGrouped(ext[0] < 16 || ext[jB] < 16, false)) // (the plain tiles need 16 and more)
+        // (the plain tiles need 16 and more; and up to 2^23 f16 they make too few workgroups, where grouped ones are cut
+        // until they make enough: 692 x 464 10.1 us in tiles, 4.2 grouped, 691 x 4279 11.8 and 7.2, 123 x 40061 11.1 and 10.2)
+        else if(tune.tile < 0
+                && tryGrouped(ext[0] < 16 || ext[jB] < 16 || (tune.kernel < 0 && in.elem_bytes == 2 && count <= (1 << 23) && (count >= (1 << 18) || !whole)), false))
             return PermuteStatus::OK;
         else
+        {
             kernel = (ext[0] >= 16 && ext[jB] >= 16) ? HIPTK_PERM_TILED : HIPTK_PERM_GATHER;
+            // blocks transposed in place, which no tile can be put together from: one thread per element reads and writes
+            // them from the caches (f16 19.25.23.8.29 -> (1,0,4,2,3) 66 us in tiles, 7.8 here; f32 19.25.230.29 21 and 10)
+            const int    order[] = {0, 1, 2};
+            const Tile   t       = (in.elem_bytes == 4 ? TILES4 : TILES2)[pickTile(in.elem_bytes, ext[0], ext[jB], order)];
+            const double inside  = coverage(ext[0], t.ti) * coverage(ext[jB], t.tj);
+            if(tune.kernel < 0 && tune.tile < 0 && inside < 0.15)
+                kernel = HIPTK_PERM_GATHER;
+        }
         out.kernel = kernel;
         if(kernel == HIPTK_PERM_GATHER)
             return PermuteStatus::OK;
@@ -393,6 +421,8 @@ namespace hipta
         if(kernel == HIPTK_PERM_TILED)
         {
             out.mode_j = jB;
+            // (sixteen tiles along j before the next along i: with each die taking neighbouring tiles 0.97 of the time of one)
+            out.group = tune.group >= 0 ? tune.group : 16;
             std::vector<int64_t> bOthers;
             for(int d = 0; d < r; ++d)
                 if(d != jB)
@@ -404,13 +434,30 @@ namespace hipta
             // The 64 KiB tile doubles the contiguous run (on both sides for f32: 512 bytes; on A's
             // side for f16), which HBM rewards as long as the tile grid does not lose much more
             // of it at the edges.
+            // (and it leaves workgroups enough: f32 5128 x 880 12.2 us in 287 tiles of 64 KiB, 9.1 in small ones, but 729.42.226
+            // -> (2,0,1) 14.6 in 504 and 19.3)
             if(tune.tile < 0)
             {
-                const Tile*  ts   = in.elem_bytes == 4 ? TILES4 : TILES2;
-                const double cur  = coverage(ext[0], ts[out.tile].ti) * coverage(ext[jB], ts[out.tile].tj);
-                const double big  = coverage(ext[0], ts[3].ti) * coverage(ext[jB], ts[3].tj);
-                if(big >= 0.9 * cur)
-                    out.tile = 3;
+                const Tile*   ts    = in.elem_bytes == 4 ? TILES4 : TILES2;
+                const double  cur   = coverage(ext[0], ts[out.tile].ti) * coverage(ext[jB], ts[out.tile].tj);
+                const double  big   = coverage(ext[0], ts[3].ti) * coverage(ext[jB], ts[3].tj);
+                const int64_t tiles = ((ext[0] + ts[3].ti - 1) / ts[3].ti) * ((ext[jB] + ts[3].tj - 1) / ts[3].tj) * (count / (ext[0] * ext[jB]));
+                const double  sq    = coverage(ext[0], ts[0].ti) * coverage(ext[jB], ts[0].tj);
+                if(smallStrip)
+                    out.tile = 0;
+                else if(big >= 0.9 * cur)
+                    out.tile = tiles >= 384 || sq < 0.8 * cur ? 3 : 0;
+            }
+            // Narrow vectors are bound by the number of accesses: 16-byte ones at any element instead (those at the end of a
+            // line moved back to end with it), for single f16 and for f32 that is read in less (f16 2712 x 81993 230 -> 218
+            // us, 1943.205.637 -> (2,1,0) 460 -> 261, 4459 x 2670 26.0 -> 18.1; f32 2073.32.279 -> (2,1,0) 42.9 -> 37.6).  Not
+            // for pairs of f16 (324.350.368 -> (1,2,0) 49 -> 61) nor f32 read whole (164.329.609 -> (1,0,2) 62.8 -> 66.7).
+            // (Narrow for the extents' sake: a base off its alignment alone keeps the vectors it admits.)
+            if(const int er = pickVec(in.elem_bytes, full, ext[0], aOthers, nullptr, false), ew = pickVec(in.elem_bytes, full, ext[jB], bOthers, nullptr, false);
+               tune.loose || (cap >= full && tune.kernel < 0 && (in.elem_bytes == 2 ? std::min(er, ew) == 1 : er < full)))
+            {
+                out.loose = 1;
+                out.vec_r = out.vec_w = full;
             }
         }
         else
@@ -464,6 +511,56 @@ namespace hipta
                 out.tile   = 0;
                 out.vec_r = out.vec_w = full;
             }
+        }
+        return PermuteStatus::OK;
+    }
+
+    PermuteStatus plan_permutation(const PermuteIn& in, const PermuteTuning& tune, hiptk_permute_t& out)
+    {
+        const PermuteStatus st = pick_kernel(in, tune, out);
+        if(st != PermuteStatus::OK)
+            return st;
+        // Runs of B that do not start at the 64 bytes memory is written in: two tiles each write a part of the lines at
+        // their edges, which reach memory whole only if both parts meet in one die's cache.  So neighbouring tiles go to
+        // one die (`bands`) and their stores are ordinary ones (`keep`): f32 946.579.437 -> (2,1,0) 762 -> 467 us,
+        // 2073.32.279 -> (2,1,0) 94 -> 43, f16 2712 x 81993 390 -> 230.
+        int64_t count = 1, runs64 = 1;
+        int     jB    = 0;
+        for(int d = 0; d < out.rank; ++d)
+        {
+            count *= out.extent[d];
+            if(out.b_stride[d] == 1)
+                jB = d;
+        }
+        for(int d = 0; d < out.rank; ++d)
+            if(d != jB && out.b_stride[d] * (int64_t)out.elem_bytes % 64 != 0)
+                runs64 = 0;
+        // (blocks transposed in place share no line with another tile's block that ordinary stores could put together: f16
+        // 96.78.191.51 -> (1,0,2,3) 55 us, 63 with both)
+        const bool inPlace = out.rank >= 2 && jB == 1 && out.b_stride[0] == out.extent[1];
+        if(inPlace)
+            return PermuteStatus::OK;
+        const Tile* ts = out.elem_bytes == 4 ? TILES4 : TILES2;
+        switch(out.kernel)
+        {
+        case HIPTK_PERM_TILED:
+            // neighbours on one die also share what they read: 46 random shapes 0.92 of the time, aligned ones among them
+            // (f32 1 GiB 379.5 -> 371).  Ordinary stores where the runs are shorter than lines, and on tensors the caches
+            // do not hold (up to there they cost 5-10 %: f32 3607 x 590 7.8 -> 8.5, 2307 x 2322 11.8 -> 12.9).
+            out.bands = 1;
+            out.keep  = !runs64
+                       && (ts[out.tile].tj * out.elem_bytes <= 128 || (count >= (1 << 23) && out.vec_w * out.elem_bytes < 16)
+                           || count >= (1 << 24) || (out.loose && out.elem_bytes == 2));
+            break;
+        case HIPTK_PERM_GROUPED:
+            // 30 random shapes 0.91 of the time on neighbouring tiles (f32 8.57.15.7.55.66 -> (5,4,2,3,1,0) 490 -> 323, 1.02
+            // at the worst), 0.90 with ordinary stores besides
+            out.bands = 1;
+            out.keep  = !runs64;
+            break;
+        // (strips and shared tiles with both: 0.98 and 0.96 over 29 shapes, and the choice between two stores costs small
+        // ones up to 11 %, f16 45.625.454 -> (1,2,0) 15.5 -> 17.3)
+        default: break;
         }
         return PermuteStatus::OK;
     }

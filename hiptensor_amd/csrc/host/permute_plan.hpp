@@ -38,6 +38,8 @@ namespace hipta
         int tile    = -1; // 0..2, -1: automatic
         int max_vec = 8; // cap on elements per load / store
         int group   = -1; // tiles per band of the workgroup order, -1: automatic
+        bool gather = true; // small tensors may go one thread per element
+        bool loose  = false; // with HIPTK_PERM_TILED: 16-byte vectors at any element whatever the extents
     };
 
     // Fills `out` (alpha and the operators are left for the caller); out.rank is the number of

@@ -85,7 +85,10 @@ namespace hipta
             const uintptr_t alignA = std::max<uintptr_t>(t.align ? t.align : (uintptr_t)elem_bytes, (uintptr_t)pin.elem_bytes);
             pin.A                  = reinterpret_cast<const void*>(alignA);
             pin.B                  = reinterpret_cast<const void*>((uintptr_t)PACK_ALIGN);
-            if(plan_permutation(pin, PermuteTuning{}, po.perm) != PermuteStatus::OK)
+            // (vectors also for small operands: one below its declared alignment is refused at the launch, whatever its size)
+            PermuteTuning tune;
+            tune.gather = false;
+            if(plan_permutation(pin, tune, po.perm) != PermuteStatus::OK)
                 return false;
             if(po.perm.rank < 2)
                 return false; // already in that order: nothing a copy would change

@@ -125,6 +125,82 @@ namespace hiptk
         return r;
     }
 
+    // ---------------------------------------------------------------- plain tiles (HIPTK_PERM_TILED)
+
+    // The part of the work workgroup `b` of `n` takes: with `bands`, workgroups of one die (ids that are congruent mod 8)
+    // take neighbouring parts.
+    HIPTK_PERM_FN uint32_t tile_work(uint32_t b, uint32_t n, bool bands)
+    {
+        if(!bands)
+            return b;
+        const uint32_t die = b & 7, rem = n & 7;
+        return die * (n >> 3) + (die < rem ? die : rem) + (b >> 3);
+    }
+
+    // First element along both tile modes of the work-th tile, and its offsets in A and B.
+    // Workgroups that run at the same time should spread over both tile modes: tiles that are neighbours along i touch
+    // neighbouring addresses of A, neighbours along j neighbouring addresses of B.  The tile plane is cut into bands of
+    // `group` tiles along j; inside a band the walk is j-first.
+    template <typename Args>
+    HIPTK_PERM_FN void tile_origin(const Args& a, uint32_t work, uint32_t TI, uint32_t TJ, uint32_t& i0, uint32_t& j0, uint32_t& aoff, uint32_t& boff)
+    {
+        const uint32_t plane = a.nt_i * a.nt_j;
+        uint32_t       blk   = work / plane;
+        const uint32_t lin   = work - blk * plane;
+        uint32_t       ti, tj;
+        if(a.group == 0)
+        {
+            // diagonal walk: consecutive workgroups differ in both tile coordinates, so that
+            // with power-of-two strides neither side keeps hitting the same memory channels
+            ti                = lin % a.nt_i;
+            const uint32_t rj = lin / a.nt_i;
+            tj                = (rj + ti) % a.nt_j;
+        }
+        else
+        {
+            const uint32_t band = lin / (a.group * a.nt_i);
+            const uint32_t rem  = lin - band * (a.group * a.nt_i);
+            const uint32_t left = a.nt_j - band * a.group;
+            const uint32_t rows = left < a.group ? left : a.group;
+            ti                  = rem / rows;
+            tj                  = band * a.group + (rem - ti * rows);
+        }
+        aoff = 0;
+        boff = 0;
+        for(int d = 0; d < a.nb; ++d)
+        {
+            const uint32_t c = blk % a.bext[d];
+            blk /= a.bext[d];
+            aoff += c * a.ba[d];
+            boff += c * a.bb[d];
+        }
+        i0 = ti * TI;
+        j0 = tj * TJ;
+        aoff += i0 + j0 * a.a_j;
+        boff += i0 * a.b_i + j0 * a.b_j;
+    }
+
+    // Vector v of a tile's `lines` rows (columns) of n elements, W elements of `per_line` vectors a line: the line and the
+    // first element along it.
+    struct TileVector
+    {
+        bool     ok; // inside the tile
+        uint32_t line, at;
+    };
+
+    // (LOOSE: the last vector of a line is moved back to end with it; n is W at least)
+    template <int W, bool LOOSE>
+    HIPTK_PERM_FN TileVector tile_vector(uint32_t v, uint32_t per_line, uint32_t n, uint32_t lines)
+    {
+        TileVector r;
+        r.line = v / per_line;
+        r.at   = (v - r.line * per_line) * W;
+        r.ok   = r.at < n && r.line < lines;
+        if(LOOSE)
+            r.at = r.at + W > n ? n - W : r.at;
+        return r;
+    }
+
     // ---------------------------------------------------------------- grouped tiles (HIPTK_PERM_GROUPED)
 
     struct GroupShape

@@ -51,6 +51,8 @@ namespace hiptk
             uint32_t    b_i, b_j; // B strides (TILED: b_j == 1, ROWS: b_i == 1)
             uint32_t    nt_i, nt_j; // tiles along i and j
             uint32_t    group; // tile order: bands of `group` tiles along j, walked j-first
+            int32_t     bands; // 1: each die takes neighbouring tiles (tile_work)
+            int32_t     keep; // 1: ordinary stores, so that the caches put lines of two tiles together
             int32_t     nb; // modes that only pick the tile's base
             uint32_t    bext[PERM_BATCH], ba[PERM_BATCH], bb[PERM_BATCH];
             float       alpha;
@@ -159,10 +161,15 @@ namespace hiptk
             return y;
         }
 
+        // Bound by HBM where runs are whole lines, and by the number of accesses and by lines written in two parts where they
+        // are not.  LOOSE: 16-byte vectors at any element on both sides.  `bands` and `keep` (set by the planner, with the
+        // reasons): tiles that share lines meet in one cache, which puts the lines together.  The three together, f16
+        // 1943.205.637 -> (2,1,0) 510 -> 262 us, 505.606.133 -> (2,0,1) 104 -> 39, f32 946.579.437 -> (2,1,0) 762 -> 483; bands
+        // alone, f32 1 GiB in whole lines 376 -> 367.5 (5.84 TB/s).
         // The tile in LDS is [TJ][TI].  Column reads must spread over the 64 banks: the small
         // tiles pad each row by one element; the 64 KiB tiles have no room for padding and XOR
         // the column index with the row number instead (in units of one 32-bit word).
-        template <typename T, int TI, int TJ, int VR, int VW, bool TRANSPOSE, int NT = PERM_THREADS, bool SWZ = false>
+        template <typename T, int TI, int TJ, int VR, int VW, bool TRANSPOSE, bool LOOSE = false, int NT = PERM_THREADS, bool SWZ = false>
         __global__ __launch_bounds__(NT) void permute_tile_kernel(PArgs a)
         {
             constexpr int PITCH = SWZ ? TI : TI + 4 / (int)sizeof(T); // an odd number of 32-bit words
@@ -170,6 +177,7 @@ namespace hiptk
             constexpr int NRV   = VPR * TJ / NT; // vectors per thread, read side
             static_assert(TI % VR == 0 && (VPR * TJ) % NT == 0 && NRV >= 1, "read shape");
             static_assert(!SWZ || TI * sizeof(T) >= 256, "a swizzled row spans all 64 banks");
+            static_assert(!LOOSE || TRANSPOSE, "rows have the linear kernel for that");
             __shared__ T tile[TRANSPOSE ? TJ * PITCH : 1];
             auto         at = [](uint32_t j, uint32_t i) -> uint32_t {
                 return SWZ ? j * TI + (i ^ ((j & 63u) * (4u / sizeof(T)))) : j * PITCH + i;
@@ -179,75 +187,55 @@ namespace hiptk
             T* __restrict__ B       = static_cast<T*>(a.B);
             const int tid           = threadIdx.x;
 
-            // Workgroups that run at the same time should spread over both tile modes: tiles that
-            // are neighbours along i touch neighbouring addresses of A, neighbours along j
-            // neighbouring addresses of B.  The tile plane is cut into bands of `group` tiles
-            // along j; inside a band the walk is j-first.
-            const uint32_t plane = a.nt_i * a.nt_j;
-            uint32_t       blk   = blockIdx.x / plane;
-            const uint32_t lin   = blockIdx.x - blk * plane;
-            uint32_t ti, tj;
-            if(a.group == 0)
-            {
-                // diagonal walk: consecutive workgroups differ in both tile coordinates, so that
-                // with power-of-two strides neither side keeps hitting the same memory channels
-                ti                = lin % a.nt_i;
-                const uint32_t rj = lin / a.nt_i;
-                tj                = (rj + ti) % a.nt_j;
-            }
-            else
-            {
-                const uint32_t band = lin / (a.group * a.nt_i);
-                const uint32_t rem  = lin - band * (a.group * a.nt_i);
-                const uint32_t left = a.nt_j - band * a.group;
-                const uint32_t rows = left < a.group ? left : a.group;
-                ti                  = rem / rows;
-                tj                  = band * a.group + (rem - ti * rows);
-            }
-            uint32_t       aoff = 0, boff = 0;
-            for(int d = 0; d < a.nb; ++d)
-            {
-                const uint32_t c = blk % a.bext[d];
-                blk /= a.bext[d];
-                aoff += c * a.ba[d];
-                boff += c * a.bb[d];
-            }
-            const uint32_t i0 = ti * TI, j0 = tj * TJ;
-            aoff += i0 + j0 * a.a_j;
-            boff += i0 * a.b_i + j0 * a.b_j;
+            uint32_t i0, j0, aoff, boff;
+            tile_origin(a, tile_work(blockIdx.x, gridDim.x, a.bands != 0), TI, TJ, i0, j0, aoff, boff);
+            // the part of the tile inside the extents
+            const uint32_t nx = a.e_i - i0 < TI ? a.e_i - i0 : TI, ny = a.e_j - j0 < TJ ? a.e_j - j0 : TJ;
 
             const T alpha = static_cast<T>(a.alpha);
 
-            Vec<T, VR> r[NRV];
-#pragma unroll
-            for(int k = 0; k < NRV; ++k)
+            if(!LOOSE || nx >= VR)
             {
-                // Lanes outside the extents load the tile's first element instead of branching
-                // around the load: a branch per load would make the compiler wait for each load
-                // before issuing the next, and the loads must all be in flight together.
-                const uint32_t v = tid + k * NT, iv = v % VPR, j = v / VPR;
-                const bool     ok = (i0 + iv * VR < a.e_i) && (j0 + j < a.e_j);
-                r[k] = load_stream<T, VR>(A + aoff + (ok ? iv * VR + j * a.a_j : 0u));
-            }
+                Vec<T, VR> r[NRV];
 #pragma unroll
-            for(int k = 0; k < NRV; ++k)
-            {
-                const uint32_t v = tid + k * NT, iv = v % VPR, j = v / VPR;
-#pragma unroll
-                for(int e = 0; e < VR; ++e)
-                    r[k].v[e] = element_op(r[k].v[e], alpha, a.op_a, a.op_b);
-                if constexpr(TRANSPOSE)
+                for(int k = 0; k < NRV; ++k)
                 {
+                    // Lanes outside the extents load the tile's first element instead of branching
+                    // around the load: a branch per load would make the compiler wait for each load
+                    // before issuing the next, and the loads must all be in flight together.
+                    const TileVector v    = tile_vector<VR, LOOSE>(tid + k * NT, VPR, nx, ny);
+                    const T*         from = A + aoff + (v.ok ? v.at + v.line * a.a_j : 0u);
+                    if constexpr(LOOSE)
+                        r[k] = load_loose(from);
+                    else
+                        r[k] = load_stream<T, VR>(from);
+                }
+#pragma unroll
+                for(int k = 0; k < NRV; ++k)
+                {
+                    const TileVector v = tile_vector<VR, LOOSE>(tid + k * NT, VPR, nx, ny);
 #pragma unroll
                     for(int e = 0; e < VR; ++e)
-                        tile[at(j, iv * VR + e)] = r[k].v[e];
+                        r[k].v[e] = element_op(r[k].v[e], alpha, a.op_a, a.op_b);
+                    if constexpr(TRANSPOSE)
+                    {
+                        if(!LOOSE || v.ok)
+#pragma unroll
+                            for(int e = 0; e < VR; ++e)
+                                tile[at(v.line, v.at + e)] = r[k].v[e];
+                    }
+                    else
+                    {
+                        if(v.ok)
+                            store_stream<T, VR>(B + boff + v.at + v.line * a.b_j, r[k]);
+                    }
                 }
-                else
-                {
-                    const bool ok = (i0 + iv * VR < a.e_i) && (j0 + j < a.e_j);
-                    if(ok)
-                        store_stream<T, VR>(B + boff + iv * VR + j * a.b_j, r[k]);
-                }
+            }
+            else
+            {
+                // (the last tile of an extent that leaves it less than a vector)
+                for(uint32_t u = tid; u < nx * ny; u += NT)
+                    tile[at(u / nx, u % nx)] = element_op(A[aoff + u % nx + u / nx * a.a_j], alpha, a.op_a, a.op_b);
             }
             if constexpr(TRANSPOSE)
             {
@@ -255,18 +243,36 @@ namespace hiptk
                 constexpr int NWV = VPC * TI / NT;
                 static_assert(TJ % VW == 0 && (VPC * TI) % NT == 0 && NWV >= 1, "write shape");
                 __syncthreads();
+                auto write = [&](auto keep_c) {
 #pragma unroll
-                for(int k = 0; k < NWV; ++k)
+                    for(int k = 0; k < NWV; ++k)
+                    {
+                        const TileVector v = tile_vector<VW, LOOSE>(tid + k * NT, VPC, ny, nx);
+                        Vec<T, VW>       o;
+#pragma unroll
+                        for(int e = 0; e < VW; ++e)
+                            o.v[e] = tile[at(v.at + e, v.line)];
+                        T* to = B + boff + v.at + v.line * a.b_i;
+                        if(v.ok)
+                        {
+                            if constexpr(decltype(keep_c)::value)
+                                __builtin_memcpy(to, &o, sizeof(o));
+                            else if constexpr(LOOSE)
+                                store_loose(to, o);
+                            else
+                                store_stream<T, VW>(to, o);
+                        }
+                    }
+                };
+                if(LOOSE && ny < VW)
                 {
-                    const uint32_t v = tid + k * NT, jv = v % VPC, i = v / VPC;
-                    const bool     ok = (j0 + jv * VW < a.e_j) && (i0 + i < a.e_i);
-                    Vec<T, VW>     o;
-#pragma unroll
-                    for(int e = 0; e < VW; ++e)
-                        o.v[e] = tile[at(jv * VW + e, i)];
-                    if(ok)
-                        store_stream<T, VW>(B + boff + jv * VW + i * a.b_i, o);
+                    for(uint32_t u = tid; u < nx * ny; u += NT)
+                        B[boff + u % ny + u / ny * a.b_i] = tile[at(u % ny, u / ny)];
                 }
+                else if(a.keep)
+                    write(std::integral_constant<bool, true>{});
+                else
+                    write(std::integral_constant<bool, false>{});
             }
         }
 
@@ -439,6 +445,7 @@ namespace hiptk
             GroupShape  s;
             const void* A;
             void*       B;
+            int32_t     bands, keep; // as in PArgs
             float       alpha;
             int32_t     op_a, op_b;
         };
@@ -466,7 +473,7 @@ namespace hiptk
             T* __restrict__ B       = static_cast<T*>(a.B);
             const uint32_t tid      = threadIdx.x;
 
-            const GroupTile t     = group_tile(a.s, blockIdx.x);
+            const GroupTile t     = group_tile(a.s, tile_work(blockIdx.x, gridDim.x, a.bands != 0));
             const uint32_t  RV    = group_per_line(a.s.w_i * a.s.c_i, VR, LOOSE), CV = group_per_line(a.s.w_j * a.s.c_j, VW, LOOSE);
             const T         alpha = static_cast<T>(a.alpha);
 
@@ -501,7 +508,7 @@ namespace hiptk
                     }
                 }
             };
-            auto write = [&](auto width, uint32_t per_col, uint32_t m_col) {
+            auto write = [&](auto width, auto keep_c, uint32_t per_col, uint32_t m_col) {
                 constexpr int  W     = decltype(width)::value;
                 const uint32_t total = per_col * t.nx;
                 for(uint32_t v = tid; v < total; v += NT)
@@ -514,7 +521,9 @@ namespace hiptk
                         for(int e = 0; e < W; ++e)
                             o.v[e] = tile[(g.at + e) * a.s.pitch + g.line];
                         T* to = B + t.boff + g.at + g.off;
-                        if constexpr(LOOSE && W > 1)
+                        if constexpr(decltype(keep_c)::value)
+                            __builtin_memcpy(to, &o, sizeof(o));
+                        else if constexpr(LOOSE && W > 1)
                             store_loose(to, o);
                         else
                             store_stream<T, W>(to, o);
@@ -527,10 +536,13 @@ namespace hiptk
             else
                 read(One{}, group_singles(t.nx), recip(group_singles(t.nx)));
             __syncthreads();
-            if(!LOOSE || t.ny >= VW)
-                write(std::integral_constant<int, VW>{}, CV, a.s.m_cv);
+            typedef std::integral_constant<bool, true> Keep;
+            if(LOOSE && t.ny < VW)
+                write(One{}, Keep{}, group_singles(t.ny), recip(group_singles(t.ny)));
+            else if(a.keep)
+                write(std::integral_constant<int, VW>{}, Keep{}, CV, a.s.m_cv);
             else
-                write(One{}, group_singles(t.ny), recip(group_singles(t.ny)));
+                write(std::integral_constant<int, VW>{}, std::integral_constant<bool, false>{}, CV, a.s.m_cv);
         }
 
         struct HArgs
@@ -752,24 +764,26 @@ namespace hiptk
         constexpr TileShape TILES4[NUM_TILES] = {{64, 64}, {256, 16}, {16, 256}, {128, 128}};
         constexpr TileShape TILES2[NUM_TILES] = {{128, 128}, {512, 32}, {32, 512}, {256, 128}};
 
-        template <typename T, int TI, int TJ, int VR, int VW, bool TR, bool BIG>
+        template <typename T, int TI, int TJ, int VR, int VW, bool TR, bool BIG, bool LOOSE = false>
         int launch_tile(const PArgs& a, uint32_t grid, hipStream_t s)
         {
             if constexpr(BIG)
             {
                 if constexpr(TR)
-                    hipLaunchKernelGGL((permute_tile_kernel<T, TI, TJ, VR, VW, true, 512, true>), dim3(grid), dim3(512), 0, s, a);
+                    hipLaunchKernelGGL((permute_tile_kernel<T, TI, TJ, VR, VW, true, LOOSE, 512, true>), dim3(grid), dim3(512), 0, s, a);
                 else
                     return -1;
             }
             else
-                hipLaunchKernelGGL((permute_tile_kernel<T, TI, TJ, VR, VW, TR>), dim3(grid), dim3(PERM_THREADS), 0, s, a);
+                hipLaunchKernelGGL((permute_tile_kernel<T, TI, TJ, VR, VW, TR, LOOSE>), dim3(grid), dim3(PERM_THREADS), 0, s, a);
             return (int)hipGetLastError();
         }
 
         template <typename T, int TI, int TJ, int VMAX, bool BIG = false>
-        int launch_tile_vec(bool transpose, int vr, int vw, const PArgs& a, uint32_t grid, hipStream_t s)
+        int launch_tile_vec(bool transpose, bool loose, int vr, int vw, const PArgs& a, uint32_t grid, hipStream_t s)
         {
+            if(loose)
+                return launch_tile<T, TI, TJ, VMAX, VMAX, true, BIG, true>(a, grid, s);
 #define HIPTK_PERM_CASE(R, W)                                                   \
     if(vr == R && vw == W)                                                      \
         return transpose ? launch_tile<T, TI, TJ, R, W, true, BIG>(a, grid, s)   \
@@ -788,15 +802,15 @@ namespace hiptk
         }
 
         template <typename T, int VMAX>
-        int launch_tile_shape(int tile, bool transpose, int vr, int vw, const PArgs& a, uint32_t grid, hipStream_t s)
+        int launch_tile_shape(int tile, bool transpose, bool loose, int vr, int vw, const PArgs& a, uint32_t grid, hipStream_t s)
         {
             constexpr const TileShape* TS = sizeof(T) == 4 ? TILES4 : TILES2;
             switch(tile)
             {
-            case 0: return launch_tile_vec<T, TS[0].ti, TS[0].tj, VMAX>(transpose, vr, vw, a, grid, s);
-            case 1: return launch_tile_vec<T, TS[1].ti, TS[1].tj, VMAX>(transpose, vr, vw, a, grid, s);
-            case 2: return launch_tile_vec<T, TS[2].ti, TS[2].tj, VMAX>(transpose, vr, vw, a, grid, s);
-            case 3: return launch_tile_vec<T, TS[3].ti, TS[3].tj, VMAX, true>(transpose, vr, vw, a, grid, s);
+            case 0: return launch_tile_vec<T, TS[0].ti, TS[0].tj, VMAX>(transpose, loose, vr, vw, a, grid, s);
+            case 1: return launch_tile_vec<T, TS[1].ti, TS[1].tj, VMAX>(transpose, loose, vr, vw, a, grid, s);
+            case 2: return launch_tile_vec<T, TS[2].ti, TS[2].tj, VMAX>(transpose, loose, vr, vw, a, grid, s);
+            case 3: return launch_tile_vec<T, TS[3].ti, TS[3].tj, VMAX, true>(transpose, loose, vr, vw, a, grid, s);
             default: return -1;
             }
         }
@@ -1000,7 +1014,7 @@ extern "C" const char* hiptk_permute_kernel_name(const hiptk_permute_t* p)
         const TileShape t = (p->elem_bytes == 4 ? TILES4 : TILES2)[p->tile];
         snprintf(name,
                  sizeof(name),
-                 "permute_%s_%s_%dx%d_r%d_w%d",
+                 p->kernel == HIPTK_PERM_TILED && p->loose ? "permute_%s_%s_%dx%d_r%d_w%d_loose" : "permute_%s_%s_%dx%d_r%d_w%d",
                  p->kernel == HIPTK_PERM_TILED ? "tiled" : "rows",
                  type_tag(p->elem_bytes),
                  t.ti,
@@ -1157,18 +1171,25 @@ extern "C" int hiptk_permute(const hiptk_permute_t* p, const void* A, void* B, v
             return HIPTK_ERR_ARG;
         // what the vector widths assume: whole vectors inside the extents, every other
         // stride and both base pointers multiples of the vector
-        const int vr = p->vec_r, vw = p->vec_w;
-        if(p->extent[0] % vr != 0 || !aligned(A, vr * p->elem_bytes))
+        // (loose: 16 bytes at any element)
+        const int  vr = p->vec_r, vw = p->vec_w;
+        const bool loose = transpose && p->loose != 0;
+        const int  wmode = transpose ? mj : 0; // the mode stores run along
+        if(loose && (vr * p->elem_bytes != 16 || vw != vr))
             return HIPTK_ERR_ARG;
-        for(int d = 1; d < p->rank; ++d)
-            if(p->a_stride[d] % vr != 0)
+        if(!loose)
+        {
+            if(p->extent[0] % vr != 0 || !aligned(A, vr * p->elem_bytes))
                 return HIPTK_ERR_ARG;
-        const int wmode = transpose ? mj : 0; // the mode stores run along
-        if(p->extent[wmode] % vw != 0 || !aligned(B, vw * p->elem_bytes))
-            return HIPTK_ERR_ARG;
-        for(int d = 0; d < p->rank; ++d)
-            if(d != wmode && p->b_stride[d] % vw != 0)
+            for(int d = 1; d < p->rank; ++d)
+                if(p->a_stride[d] % vr != 0)
+                    return HIPTK_ERR_ARG;
+            if(p->extent[wmode] % vw != 0 || !aligned(B, vw * p->elem_bytes))
                 return HIPTK_ERR_ARG;
+            for(int d = 0; d < p->rank; ++d)
+                if(d != wmode && p->b_stride[d] % vw != 0)
+                    return HIPTK_ERR_ARG;
+        }
 
         const TileShape t = (p->elem_bytes == 4 ? TILES4 : TILES2)[p->tile];
         PArgs           a;
@@ -1183,6 +1204,8 @@ extern "C" int hiptk_permute(const hiptk_permute_t* p, const void* A, void* B, v
         a.nt_i  = (a.e_i + t.ti - 1) / t.ti;
         a.nt_j  = (a.e_j + t.tj - 1) / t.tj;
         a.group = p->group == 0 ? 0u : (uint32_t)std::max(1, std::min(p->group, (int32_t)a.nt_j));
+        a.bands = p->bands != 0;
+        a.keep  = p->keep != 0;
         a.alpha = p->alpha;
         a.op_a  = p->op_a;
         a.op_b  = p->op_b;
@@ -1199,8 +1222,8 @@ extern "C" int hiptk_permute(const hiptk_permute_t* p, const void* A, void* B, v
         }
         if(grid >= (int64_t(1) << 31))
             return HIPTK_ERR_ARG;
-        rc = p->elem_bytes == 4 ? launch_tile_shape<float, 4>(p->tile, transpose, vr, vw, a, (uint32_t)grid, s)
-                                : launch_tile_shape<_Float16, 8>(p->tile, transpose, vr, vw, a, (uint32_t)grid, s);
+        rc = p->elem_bytes == 4 ? launch_tile_shape<float, 4>(p->tile, transpose, loose, vr, vw, a, (uint32_t)grid, s)
+                                : launch_tile_shape<_Float16, 8>(p->tile, transpose, loose, vr, vw, a, (uint32_t)grid, s);
     }
     else if(p->kernel == HIPTK_PERM_GROUPED)
     {
@@ -1252,6 +1275,8 @@ extern "C" int hiptk_permute(const hiptk_permute_t* p, const void* A, void* B, v
             return HIPTK_ERR_ARG; // (the reciprocals are exact for divisors of 2 and more)
         int64_t grid = 0;
         a.s          = group_shape(*p, grid);
+        a.bands      = p->bands != 0;
+        a.keep       = p->keep != 0;
         a.alpha      = p->alpha;
         a.op_a       = p->op_a;
         a.op_b       = p->op_b;

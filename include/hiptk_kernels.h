@@ -240,8 +240,11 @@ typedef struct hiptk_permute
     int32_t mode_i2, mode_j2; /* GROUPED: the second row / column mode, or -1                     */
     int32_t chunk_i, chunk_j; /* GROUPED: indices of mode_i2 / mode_j2 per tile (1 when absent)   */
     int32_t width_i, width_j; /* GROUPED: elements of mode 0 / mode_j per tile                    */
-    int32_t loose; /* GROUPED: 16-byte vectors that start at any element and need divide nothing
+    int32_t loose; /* GROUPED, TILED: 16-byte vectors that start at any element and need divide nothing
                       (vec_r == vec_w == 16 / elem_bytes)                                         */
+    int32_t bands; /* TILED / GROUPED: 1: each die takes neighbouring tiles                       */
+    int32_t keep;  /* TILED / GROUPED: 1: B is written with ordinary stores instead of non-temporal ones (runs of
+                      B that start inside a line: two tiles write parts of it)                    */
 } hiptk_permute_t;
 
 /* Name of the kernel a problem selects ("" if the combination is not instantiated). */
