@@ -174,6 +174,17 @@ namespace hipta
         {
             return c.split_k > 1 && !c.sol->direct && (std::min(v.x_vec, v.y_vec) > 1 || c.split_k >= 64) ? c.est_us - std::min(6.0, 1.5 + 0.16 * c.split_k) : c.est_us;
         }
+
+        // ... of a plan on packed copies.  (8-byte elements: without the tiles that take operands at any element, which a copy of odd
+        // extents would run.  The element-by-element gather it saves there is within 13 % of whole vectors, less than the estimates
+        // of the moves and of those tiles are good for.)
+        double packed_us(const std::vector<Choice>& ranked, const GemmView& v)
+        {
+            for(const Choice& c : ranked)
+                if(!(v.elem_bytes == 8 && c.sol->direct && c.sol->tile_id >= 4))
+                    return comparable_us(c, v);
+            return comparable_us(ranked.front(), v);
+        }
     }
 
     RepackMode repack_mode_from_env()
@@ -255,7 +266,7 @@ namespace hipta
                 alt.ranked = rank_choices(candidates, alt.view, std::min(max_ws - alt.pack_bytes, split_cap), dev);
                 if(alt.ranked.empty())
                     continue;
-                double us = comparable_us(alt.ranked.front(), alt.view) + alt.a.est_us + alt.b.est_us;
+                double us = packed_us(alt.ranked, alt.view) + alt.a.est_us + alt.b.est_us;
                 if(mode == RepackMode::FORCE)
                     us -= 1e9 * ((alt.a.on ? 1 : 0) + (alt.b.on ? 1 : 0)); // as many copies as the layouts admit
                 if(!have_best || us < best_us)

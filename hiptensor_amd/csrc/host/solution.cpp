@@ -247,6 +247,9 @@ namespace hipta
             if(per_cu >= 3)
                 step_us *= 1.3;
         }
+        // (tile ids 4 and 5 of the classes with more than one element per vector: operands at any element)
+        const bool any_split_lines = s.direct && s.tile_id >= 4 && class_flops_per_clk_cu(v.cls) != 4096.0 && v.cls != HIPTK_C64 && v.x_kfast && v.y_kfast
+                                     && !(v.x_lines && v.y_lines);
         if(s.direct && class_flops_per_clk_cu(v.cls) != 4096.0)
         {
             // The 32/64-bit 64 x 64 tiles whose operand tiles are loaded straight into LDS (four waves, three to
@@ -271,6 +274,14 @@ namespace hipta
             // four per CU, 92.7)
             case HIPTK_C64: r = big ? TileRate{0.85, 0.91} : TileRate{0.85, 0.70}; break;
             default: break;
+            }
+            // (the tiles that take operands at any element, on rows off the 128-byte lines along k: f32 1248 x 219 x 798 on 32 x 32
+            // 21.1 us, staged in four slices 15.9; 24 x 8746 x 5506 on 64 x 64 in eight 86.0, staged in 16 78.9)
+            if(any_split_lines)
+            {
+                const double f = v.cls == HIPTK_F32 ? (big ? 0.9 : 0.8) : 0.92;
+                r.alone *= f;
+                r.full *= f;
             }
             // ... whose prologue (tables, then the first tiles' flight) and epilogue nothing overlaps when a
             // CU runs one or two rounds of them: 2048 x 2048 x K f32 fits 13.9 us + 60.5 us per 1024 of K
@@ -309,7 +320,13 @@ namespace hipta
         if(ring_step)
             us = std::cbrt(us * us * us + std::pow(bytes / (dev.hbm_gbs * 1e3 * 0.72), 3.0));
         else
-            us = std::max(us, bytes / (dev.hbm_gbs * 1e3 * 0.6));
+        {
+            // (the 32 x 32 tiles that take operands at any element read 64 bytes of a row per K tile and wave: off the 128-byte
+            // lines, from HBM, that comes at half the rate.  f32 15015 x 36 x 7322, both k-contiguous, 295 us on them, 134 on 64 x
+            // 64; 24 x 8746 x 5506 120 and 92.  Row-contiguous, and where operands stay in the caches, they win as their
+            // rates say: 901 x 176 x 332 c32 11.0 and 25.1)
+            us = std::max(us, bytes / (dev.hbm_gbs * 1e3 * (any_split_lines && s.bp * s.bq < 4096 ? 0.32 : 0.6)));
+        }
         // split-K slices of different tiles share nothing in time: every workgroup's operand panels come through
         // the fabric (256 x 256 x 65536 f16 in 32 slices: 16 tiles of 64 x 64 move 2.7e8 B for 6.7e7 algorithmic
         // and take 40.5 us, 4 tiles of 128 x 128 move half of that and take 33.4)

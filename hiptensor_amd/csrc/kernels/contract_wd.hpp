@@ -205,11 +205,20 @@ namespace hiptk
         }
     }
 
-    // TAIL: K need not be a multiple of BK.  (The test for the short last tile is a branch in every step of the
-    // main loop, which costs 2-5 %: problems without such a tile run the instantiation without it.)
-    template <typename Tr, int BK, int NS, bool WK, bool XKF, bool YKF, bool TAIL>
-    __global__ void __launch_bounds__(256, 2) contract_wd_kernel(const KArgs a)
+    // What a K that is no multiple of BK asks of the kernel.
+    enum
     {
+        WD_WHOLE, // nothing: K is a multiple of BK
+        WD_TAIL, // the short last tile comes last.  (The test for it is a branch in every step of the main loop, which costs
+                 // 2-5 %: problems without such a tile run the instantiation without it.)
+        WD_ANY // K need not be a multiple of a k-contiguous operand's vector either, vectors start at any element, and
+               // tiles are moved back: contract_wx_kernel
+    };
+
+    template <typename Tr, int BK, int NS, bool WK, bool XKF, bool YKF, int FORM>
+    __device__ __forceinline__ void wd_body(const KArgs& a)
+    {
+        constexpr bool TAIL = FORM == WD_TAIL, ANY = FORM == WD_ANY;
         typedef WdGeom<Tr, BK, NS, WK, XKF, YKF> G;
         // with a k-contiguous operand the k-slots of one k-step are V apart in k (see wd_slot_kf), for both operands
         constexpr bool VAPART = XKF || YKF;
@@ -232,9 +241,11 @@ namespace hiptk
 
         int tp, tq, slice;
         tile_coords(a, tp, tq, slice);
-        // (no tile is moved back; a tile that overhangs P or Q reads the padding of the row tables, offset 0,
-        // and stores nothing there)
-        const int p0 = tp * G::BP, q0 = tq * G::BQ;
+        // (a tile that overhangs P or Q reads the padding of the row tables, offset 0, and stores nothing there.  WD_ANY: or
+        // is moved back to end at P or Q, where it recomputes rows of its neighbour and stores its own)
+        const int p_own = tp * G::BP, q_own = tq * G::BQ;
+        const int p0    = ANY && a.shift_p && p_own + G::BP > a.P ? a.P - G::BP : p_own;
+        const int q0    = ANY && a.shift_q && q_own + G::BQ > a.Q ? a.Q - G::BQ : q_own;
 
         int       kt_begin = slice * a.ktiles_per_split;
         int       kt_end   = kt_begin + a.ktiles_per_split;
@@ -271,8 +282,10 @@ namespace hiptk
         // 32-bit byte offset from the operand's base, kept in scalar registers
         const uint32_t xkb   = (uint32_t)ES * (uint32_t)a.xk_stride;
         const uint32_t ykb   = (uint32_t)ES * (uint32_t)a.yk_stride;
-        const int      klast = (kt_begin + nt - 1) * BK;
-        int            ko    = kt_begin * BK;
+        // (WD_ANY: the short last tile is taken first, so that no step of the main loop has to look for it)
+        const int      short_k = ANY && kt_end == kt_all && nt > 0 ? a.K % BK : 0;
+        const int      klast = short_k ? (nt > 1 ? (kt_begin + nt - 2) * BK : 0) : (kt_begin + nt - 1) * BK;
+        int            ko    = short_k && nt == 1 ? 0 : kt_begin * BK;
         int            lu    = 0; // index of the next tile to be requested
         const char*    xsrc  = (const char*)a.X + (uint64_t)((uint32_t)ko * xkb);
         const char*    ysrc  = (const char*)a.Y + (uint64_t)((uint32_t)ko * ykb);
@@ -329,6 +342,26 @@ namespace hiptk
             ysrc = (const char*)a.Y + (uint64_t)((uint32_t)ko * ykb);
         };
 
+        // WD_ANY: request the slice's short last tile into ring stage 0
+        auto issue_short = [&]() {
+            const int origin = (kt_all - 1) * BK;
+#pragma unroll
+            for(int i = 0; i < NLW; i++)
+            {
+                const int    s_ = ((WK ? 0 : wave * NLW) + i) * 64 + lane;
+                const HdSlot sx = XKF ? wd_slot_kf<G::V, ROWS>(s_) : wd_slot<G::V, ROWS>(s_);
+                const HdSlot sy = YKF ? wd_slot_kf<G::V, ROWS>(s_) : wd_slot<G::V, ROWS>(s_);
+                const int    kx = wd_short_k<G::V>(sx.k, short_k, XKF || YKF), ky = wd_short_k<G::V>(sy.k, short_k, XKF || YKF);
+                const char*  px = (const char*)a.X + (uint64_t)ES * (uint32_t)a.xp[p0 + sx.row] + (uint64_t)(uint32_t)(origin + kx) * xkb;
+                const char*  py = (const char*)a.Y + (uint64_t)ES * (uint32_t)a.yq[q0 + sy.row] + (uint64_t)(uint32_t)(origin + ky) * ykb;
+                dma_dst_at(wdx, i * 1024);
+                dma_load_at(kx != WD_ZERO ? (const void*)px : (const void*)wd_zero16);
+                dma_dst_at(wdy, i * 1024);
+                dma_load_at(ky != WD_ZERO ? (const void*)py : (const void*)wd_zero16);
+            }
+            lu++;
+        };
+
         // C and the C / D offsets of the wave tile this wave will store (with waves that split K: wave 0,
         // all of the tile), unless the launch is a split-K slice, which stores partial sums
         // (complex f64 has no registers for it: 64 for its C elements beside 96 of accumulators and 64 of operands)
@@ -337,7 +370,7 @@ namespace hiptk
         const bool             whole_k = EARLY_C && a.split_k == 1;
         const bool             storer  = !WK || wave == 0;
         if(whole_k && storer)
-            epi.fetch(a, p0 + wp * 32, q0 + wq * 32 + Tr::q_of(lane), p0, q0, lane);
+            epi.fetch(a, p0 + wp * 32, q0 + wq * 32 + Tr::q_of(lane), p_own, q_own, lane);
         // (requested before the first operand tile: loads return in order, so they are back before it)
         __builtin_amdgcn_sched_barrier(0);
 
@@ -474,9 +507,33 @@ namespace hiptk
         static_assert(NS % 2 == 0, "the register copies alternate with the ring stages");
         if(nt > 0)
         {
-            wd_static_for<NS>(issue); // tiles 0 .. NS - 1
+            // tiles 0 .. NS - 1
+            if(ANY && short_k)
+            {
+                issue_short();
+                wd_static_for<NS - 1>([&](auto i_c) { issue(std::integral_constant<int, decltype(i_c)::value + 1>{}); });
+            }
+            else
+                wd_static_for<NS>(issue);
             wd_hand_over<WK, (NS - 1) * LPT>();
             read_tile(std::integral_constant<int, 0>{}, fr[0]);
+            if(ANY && VAPART && short_k % G::V != 0)
+            {
+                // the last vector's k that the vector in front of it holds as well count once
+                const int dup = G::V - short_k % G::V;
+#pragma unroll
+                for(int ks = 0; ks < KS; ks++)
+                {
+                    const int  pos  = ((ks / G::V) * Tr::KM + kslot) * G::V + ks % G::V;
+                    const bool zero = pos / G::V == short_k / G::V && pos % G::V < dup;
+#pragma unroll
+                    for(int i = 0; i < TP; i++)
+                        fr[0].x[ks][i] = zero ? S{} : fr[0].x[ks][i];
+#pragma unroll
+                    for(int j = 0; j < TQ; j++)
+                        fr[0].y[ks][j] = zero ? S{} : fr[0].y[ks][j];
+                }
+            }
             while(t + NS <= nt)
                 wd_static_for<NS>(step);
             wd_static_for<NS - 1>([&](auto i_c) {
@@ -521,17 +578,51 @@ namespace hiptk
             if(whole_k)
                 epi.store(a, acc);
             else
-                epilogue_w<Tr, TP, TQ>(a, acc, p0, q0 + Tr::q_of(lane), p0, q0, slice, lane);
+                epilogue_w<Tr, TP, TQ>(a, acc, p0, q0 + Tr::q_of(lane), p_own, q_own, slice, lane);
         }
         else
         {
             if(whole_k)
                 epi.store(a, acc);
             else
-                epilogue_w<Tr, TP, TQ>(a, acc, p0 + wp * 32, q0 + wq * 32 + Tr::q_of(lane), p0, q0, slice, lane);
+                epilogue_w<Tr, TP, TQ>(a, acc, p0 + wp * 32, q0 + wq * 32 + Tr::q_of(lane), p_own, q_own, slice, lane);
             // the loads beyond the K range (into the spare KiB) must not outlive the workgroup's LDS
             __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
         }
+    }
+
+    template <typename Tr, int BK, int NS, bool WK, bool XKF, bool YKF, bool TAIL>
+    __global__ void __launch_bounds__(256, 2) contract_wd_kernel(const KArgs a)
+    {
+        wd_body<Tr, BK, NS, WK, XKF, YKF, TAIL ? WD_TAIL : WD_WHOLE>(a);
+    }
+
+    // The same kernel for operands at any element: vectors start anywhere (a direct load asks for 4 bytes), rows that are one
+    // ragged run have the last tile moved back, and K is any from one tile on.  Its short last tile is taken first: vectors
+    // beyond K come from zeros, and where K ends inside a vector of a k-contiguous operand, the last V k are loaded (of both
+    // operands) and those the vector in front of them holds as well are zeroed in the registers.  What such problems ran on
+    // before are the tiles staged through registers: over 38 random problems the best of these takes 0.56 of the best of those (c32
+    // 901 x 176 x 332 31.9 -> 11.0 us, f32 1617 x 1107 x 4315 195.7 -> 135.7, f64 row- by k-contiguous 258 -> 60).  Bound as
+    // contract_wd_kernel is; rows off the 128-byte lines cost it what the lines' second halves take.
+    template <typename Tr, int BK, int NS, bool WK, bool XKF, bool YKF>
+    __global__ void __launch_bounds__(256, 2) contract_wx_kernel(const KArgs a)
+    {
+        wd_body<Tr, BK, NS, WK, XKF, YKF, WD_ANY>(a);
+    }
+
+    template <typename Tr, int BK, int NS, bool WK, bool XKF, bool YKF>
+    int launch_wx(const KArgs& a, hipStream_t stream)
+    {
+        typedef WdGeom<Tr, BK, NS, WK, XKF, YKF> G;
+        if(a.K < BK || (a.shift_p && a.P < G::BP) || (a.shift_q && a.Q < G::BQ))
+            return (int)hipErrorInvalidValue;
+        auto                    kern = contract_wx_kernel<Tr, BK, NS, WK, XKF, YKF>;
+        static const hipError_t attr = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, G::LDS_BYTES);
+        if(attr != hipSuccess)
+            return (int)attr;
+        dim3 grid(a.tiles_p * a.tiles_q, 1, a.split_k);
+        hipLaunchKernelGGL(kern, grid, dim3(256), G::LDS_BYTES, stream, a);
+        return (int)hipGetLastError();
     }
 
     template <typename Tr, int BK, int NS, bool WK, bool XKF, bool YKF>
@@ -592,3 +683,15 @@ namespace hiptk
             #TR "_32x32x" #BK "_direct" #NS "k4kf" #XKF #YKF,                                       \
             &hiptk::launch_wd<hiptk::TR, BK, NS, true, XKF != 0, YKF != 0>, hiptk::TR::VMAX                     \
     }
+
+// ... and of all of these for operands at any element (contract_wx_kernel), under tile ids of their own
+#define HIPTK_WX_ENTRY(TR, ID, BK, NS, WK, XKF, YKF)                                                \
+    {                                                                                               \
+        hiptk::TR::CLS, ID, XKF, YKF, hiptk::TR::VMAX, hiptk::TR::VMAX, 1, WK ? 32 : 64, WK ? 32 : 64, BK, 256, \
+            hiptk::WdGeom<hiptk::TR, BK, NS, WK != 0, XKF != 0, YKF != 0>::LDS_BYTES,               \
+            #TR "_any_x" #BK "_ring" #NS "k4" #WK "kf" #XKF #YKF,                                   \
+            &hiptk::launch_wx<hiptk::TR, BK, NS, WK != 0, XKF != 0, YKF != 0>, 1, 0, 4              \
+    }
+#define HIPTK_WX_TILE(TR, ID, BK, NS, WK)                                                           \
+    HIPTK_WX_ENTRY(TR, ID, BK, NS, WK, 0, 0), HIPTK_WX_ENTRY(TR, ID, BK, NS, WK, 1, 1),             \
+        HIPTK_WX_ENTRY(TR, ID, BK, NS, WK, 1, 0), HIPTK_WX_ENTRY(TR, ID, BK, NS, WK, 0, 1)

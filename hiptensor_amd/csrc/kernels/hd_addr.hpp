@@ -99,6 +99,18 @@ namespace hiptk
         return kf ? k + v <= tail_k : k < tail_k;
     }
 
+    // The same tile where K may end inside a vector (contract_wx_kernel): the k (from the tile's origin, so 1 - V and up)
+    // that is loaded at its k-position k, or WD_ZERO for zeros.  With `chunks` (an operand is contiguous along k) the V
+    // positions that K ends in hold the last V k, for both operands alike.
+    constexpr int WD_ZERO = -64;
+    template <int V>
+    HIPTK_HD_FN int wd_short_k(int k, int tail_k, bool chunks)
+    {
+        if(chunks && (k | (V - 1)) >= tail_k && (k & ~(V - 1)) < tail_k)
+            return tail_k - V + (k & (V - 1));
+        return k < tail_k ? k : WD_ZERO;
+    }
+
     // ... and where the four waves of a workgroup split a slice of n K tiles between them: wave w takes
     // `count` tiles from `first` on (none, for the last waves of a short slice).
     struct WdChunk

@@ -86,6 +86,9 @@ namespace hiptk
     const KernelEntry* entries_f64(int* count);
     const KernelEntry* entries_c32(int* count);
     const KernelEntry* entries_c64(int* count);
+    const KernelEntry* entries_f32_any(int* count);
+    const KernelEntry* entries_f64_any(int* count);
+    const KernelEntry* entries_c32_any(int* count);
     const KernelEntry* entries_f64_as_f32(int* count);
     const KernelEntry* entries_f32_as_f16(int* count);
     const KernelEntry* entries_f32_as_bf16(int* count);

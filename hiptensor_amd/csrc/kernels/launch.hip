@@ -48,6 +48,9 @@ namespace hiptk
                                           entries_bf16_v2,
                                           entries_f32,
                                           entries_f64,
+                                          entries_f32_any,
+                                          entries_f64_any,
+                                          entries_c32_any,
                                           entries_c32,
                                           entries_c64,
                                           entries_f64_as_f32,
