@@ -629,14 +629,22 @@ hiptensorStatus_t hiptensorContractionGetWorkspaceSize(const hiptensorHandle_t* 
         const hipta::GemmView& v         = pc.view;
         const uint64_t         footprint = (uint64_t)(v.spanA + v.spanB + v.spanC + v.spanD) * (uint64_t)v.elem_bytes;
         const uint64_t         budget    = std::min<uint64_t>(1ull << 30, std::max<uint64_t>(64ull << 20, footprint));
-        uint64_t               need      = pc.pack_bytes + pc.ranked.front().ws_bytes;
+        // (operands declared below what the choice takes run its stand-in, which may want more slices)
+        auto wanted = [](const hipta::ContractionPlanChoice& p) {
+            uint64_t split = p.ranked.front().ws_bytes;
+            auto     below = [&](const hipta::TensorIn& t) { return t.align % (uint32_t)std::max(1, p.ranked.front().sol->vec_align) != 0; };
+            if(const hipta::Choice* o = hipta::stand_in(p.ranked.front(), p.ranked); o && (below(p.problem.A) || below(p.problem.B)))
+                split = std::max(split, o->ws_bytes);
+            return p.pack_bytes + split;
+        };
+        uint64_t need = wanted(pc);
         if(need > budget)
         {
             hipta::ContractionPlanChoice bounded;
             if(hipta::plan_contraction(in, candidatesOf(find), budget, std::min<uint64_t>(WS_CAP, budget), h->model(), hipta::repack_mode_from_env(), bounded, why)
                    == hipta::PlanStatus::OK
                && !bounded.ranked.empty())
-                need = bounded.pack_bytes + bounded.ranked.front().ws_bytes;
+                need = wanted(bounded);
             else
                 need = 0;
         }
@@ -796,8 +804,10 @@ hiptensorStatus_t hiptensorInitContractionPlan(const hiptensorHandle_t*         
         const hipta::Choice& c = ranked[pick];
         // what planning decided: requests that differ only in a workspace size that did not change
         // the decision share one state (and one set of device tables)
+        const hipta::Choice* other = hipta::stand_in(c, ranked);
         const std::string decision = problem + "|tile=" + std::to_string(c.sol->tile_id) + ",split=" + std::to_string(c.split_k) + ",pack="
-                                     + std::to_string((int)pc.a.on) + std::to_string((int)pc.b.on) + "," + std::to_string((unsigned long long)pc.pack_bytes);
+                                     + std::to_string((int)pc.a.on) + std::to_string((int)pc.b.on) + "," + std::to_string((unsigned long long)pc.pack_bytes)
+                                     + (other ? ",else=" + std::to_string(other->sol->tile_id) + "," + std::to_string(other->split_k) : std::string());
         if(PlanState* known = h->findDecision(key, decision))
         {
             st = known;
@@ -839,6 +849,11 @@ hiptensorStatus_t hiptensorInitContractionPlan(const hiptensorHandle_t*         
         p.y_rows_adjacent = v.y_rows_adjacent;
         p.xk_stride            = (int32_t)v.xk_stride;
         p.yk_stride            = (int32_t)v.yk_stride;
+        if(other)
+        {
+            p.unaligned_tile  = other->sol->tile_id;
+            p.unaligned_split = other->split_k;
+        }
         (void)hiptk_resolve(&p); // the registry is searched here, once, not at every launch
         fresh->kernel_name     = hiptk_kernel_name(&p);
         if(!h->hostOnly())
@@ -1139,7 +1154,7 @@ hiptensorStatus_t contractionImpl(const char*                       fn,
                      "KernelId: %lu KernelName: %s, %0.3f ms, %0.3f TFlops, %0.3f GB/s%s",
                      (unsigned long)st->sol->uid,
                      // (the kernel that ran: the plan's, or its register-staged stand-in for operands
-                     // that are not 16-byte aligned)
+                     // that are not aligned for it)
                      hiptk_kernel_name_at(&st->prob, X, Y),
                      ms,
                      flops / 1e9 / ms,

@@ -32,6 +32,7 @@ namespace hipta
                 s.lds_bytes = ti.lds_bytes;
                 s.direct    = ti.k_multiple > 0;
                 s.mfma_k    = ti.mfma_k;
+                s.vec_align = ti.vec_align;
                 s.name      = ti.name;
                 uint64_t h  = 0x68697074656e73ull;
                 for(uint64_t x : {(uint64_t)cls, (uint64_t)t, (uint64_t)ti.bp, (uint64_t)ti.bq, (uint64_t)ti.bk})
@@ -390,5 +391,15 @@ namespace hipta
         }
         std::stable_sort(out.begin(), out.end(), [](const Choice& a, const Choice& b) { return a.est_us < b.est_us; });
         return out;
+    }
+
+    const Choice* stand_in(const Choice& c, const std::vector<Choice>& ranked)
+    {
+        if(c.sol->vec_align == 0)
+            return nullptr;
+        for(const Choice& o : ranked)
+            if(o.sol->vec_align == 0)
+                return &o;
+        return nullptr;
     }
 }

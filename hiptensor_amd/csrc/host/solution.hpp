@@ -25,6 +25,7 @@ namespace hipta
         int         bp, bq, bk, threads, lds_bytes;
         bool        direct; // operand tiles go from global memory straight into LDS
         int         mfma_k; // 32: a 16-bit tile on v_mfma_f32_16x16x32 (else 0)
+        int         vec_align; // bytes the operands' bases must be multiples of (0: any element)
         std::string name;
     };
 
@@ -69,6 +70,10 @@ namespace hipta
                                      const GemmView&                     v,
                                      uint64_t                            max_ws,
                                      const DeviceModel&                  dev);
+
+    // What runs where an operand's base is not aligned for `c`: the best register-staged choice of the ranking that `c`
+    // comes from (nullptr: `c` takes any base, or there is none).
+    const Choice* stand_in(const Choice& c, const std::vector<Choice>& ranked);
 
     // MFMA flop per clock per CU of a class (dense peak), for estimates and reports.
     double class_flops_per_clk_cu(int cls);

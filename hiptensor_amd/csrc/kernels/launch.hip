@@ -1,5 +1,6 @@
 // Kernel-layer C ABI: kernel registry lookup, argument checks, launch, and the
 // split-K reduction kernels.
+#include <algorithm>
 #include <cstdio>
 #include <cstring>
 #include <mutex>
@@ -357,6 +358,11 @@ namespace hiptk
         {
             return e.vec_align ? e.vec_align : 16;
         }
+        // ... and what a problem's do (1, as a flag: 16)
+        int xy_aligned(const hiptk_problem_t* p)
+        {
+            return p->xy_aligned == 1 ? 16 : p->xy_aligned;
+        }
 
         // The affine-K variant is preferred when the problem allows it; the table variant
         // serves every problem.
@@ -372,7 +378,7 @@ namespace hiptk
                     if((p->shift_p && p->P < e.bp) || (p->shift_q && p->Q < e.bq))
                         continue;
                     // the direct-load kernels: a restricted K tail, vectors on multiples of 16 (or 4) bytes
-                    if(e.k_multiple > 0 && (p->K % e.k_multiple != 0 || p->K < e.bk || p->xy_aligned < vec_align(e)))
+                    if(e.k_multiple > 0 && (p->K % e.k_multiple != 0 || p->K < e.bk || xy_aligned(p) < vec_align(e)))
                         continue;
                     // ... and they address an operand with 32-bit byte offsets
                     if(e.k_multiple > 0)
@@ -392,12 +398,19 @@ namespace hiptk
             return table;
         }
 
-        // The largest register-staged tile of the problem's class and layout: what runs in place of
-        // a direct-load kernel when an operand's base address is not aligned for it.
+        // What runs in place of a direct-load kernel when an operand's base address is not aligned for it: the
+        // register-staged tile the problem names, else the largest one of its class and layout.
         const KernelEntry* staged_entry(const hiptk_problem_t* p)
         {
             const KernelEntry* best = nullptr;
             hiptk_problem_t    q    = *p;
+            if(p->unaligned_split > 0)
+            {
+                q.tile_id            = p->unaligned_tile;
+                const KernelEntry* e = find_entry(&q);
+                if(e && e->k_multiple == 0)
+                    return e;
+            }
             for(const KernelEntry& t : registry().all)
             {
                 if(t.cls != p->cls || t.k_multiple > 0)
@@ -413,15 +426,17 @@ namespace hiptk
         }
 
         // The entry a launch with these operand addresses runs: the resolved one where the plan
-        // resolved it (and the problem still is the one it was resolved for), else a search.
-        const KernelEntry* entry_for(const hiptk_problem_t* p, const void* X, const void* Y)
+        // resolved it (and the problem still is the one it was resolved for), else a search.  stands_in: it is
+        // not the plan's tile, but what runs for operands that are not aligned for that.
+        const KernelEntry* entry_for(const hiptk_problem_t* p, const void* X, const void* Y, bool& stands_in)
         {
             const KernelEntry* e = (const KernelEntry*)p->kernel;
             const bool         resolved = e && e->cls == p->cls && e->tile_id == p->tile_id && e->x_kfast == (p->x_kfast != 0)
                                   && e->y_kfast == (p->y_kfast != 0) && e->x_vec == p->x_vec && e->y_vec == p->y_vec;
             if(!resolved)
                 e = find_entry(p);
-            if(e && e->k_multiple > 0 && ((((uintptr_t)X) | ((uintptr_t)Y)) & (uintptr_t)(vec_align(*e) - 1)) != 0)
+            stands_in = e && e->k_multiple > 0 && ((((uintptr_t)X) | ((uintptr_t)Y)) & (uintptr_t)(vec_align(*e) - 1)) != 0;
+            if(stands_in)
                 e = resolved ? (const KernelEntry*)p->kernel_unaligned : staged_entry(p);
             return e;
         }
@@ -440,7 +455,8 @@ extern "C" int hiptk_resolve(hiptk_problem_t* prob)
 
 extern "C" const char* hiptk_kernel_name_at(const hiptk_problem_t* prob, const void* X, const void* Y)
 {
-    const hiptk::KernelEntry* e = prob ? hiptk::entry_for(prob, X, Y) : nullptr;
+    bool                      stands_in;
+    const hiptk::KernelEntry* e = prob ? hiptk::entry_for(prob, X, Y, stands_in) : nullptr;
     return e ? e->name : "";
 }
 
@@ -469,6 +485,7 @@ extern "C" int hiptk_tile_info(int cls, int tile_id, hiptk_tile_info_t* out)
             out->lds_bytes = e.lds_bytes;
             out->k_multiple = e.k_multiple;
             out->mfma_k     = e.mfma_k;
+            out->vec_align  = e.k_multiple > 0 ? hiptk::vec_align(e) : 0;
             std::snprintf(out->name, sizeof(out->name), "cls%d_%dx%dx%d", cls, e.bp, e.bq, e.bk);
             return HIPTK_OK;
         }
@@ -520,7 +537,8 @@ extern "C" int hiptk_contract(const hiptk_problem_t* prob,
     const bool bil = prob->op == HIPTK_OP_BILINEAR;
     if(bil && (!C || !beta || !prob->cp || !prob->cq))
         return HIPTK_ERR_ARG;
-    const KernelEntry* e = entry_for(prob, X, Y);
+    bool               stands_in = false;
+    const KernelEntry* e         = entry_for(prob, X, Y, stands_in);
     if(!e)
         return HIPTK_ERR_NO_KERNEL;
 
@@ -572,6 +590,13 @@ extern "C" int hiptk_contract(const hiptk_problem_t* prob,
     a.tiles_q  = (int32_t)((prob->Q + e->bq - 1) / e->bq);
     const int ktiles = (int)((prob->K + e->bk - 1) / e->bk);
     int       split  = prob->split_k;
+    if(stands_in && prob->unaligned_split > 0)
+    {
+        // (its slices may want more workspace than the plan asked for)
+        const uint64_t slice = (uint64_t)prob->P * (uint64_t)prob->Q * (uint64_t)acc_bytes(prob->cls);
+        const uint64_t held  = workspace ? workspace_bytes / slice : 0;
+        split                = held < (uint64_t)prob->unaligned_split ? std::max(1, (int)held) : prob->unaligned_split;
+    }
     if(split > ktiles)
         split = ktiles;
     a.ktiles_per_split = (ktiles + split - 1) / split;

@@ -65,6 +65,8 @@ typedef struct hiptk_tile_info
                            them straight into LDS: K must be a multiple of this (1: any) and at least bk,
                            and the problem xy_aligned as far as the tile asks    */
     int32_t mfma_k;     /* 32: a 16-bit tile built on v_mfma_f32_16x16x32 (else 0)   */
+    int32_t vec_align;  /* bytes that the two operands' bases must be multiples of for the tile to run (16 or 4);
+                           0: any element (tiles staged through registers)            */
 } hiptk_tile_info_t;
 
 typedef struct hiptk_problem
@@ -105,9 +107,9 @@ typedef struct hiptk_problem
     int32_t xy_aligned; /* 16 or 4: every 16-byte vector of X and Y starts a multiple of so many bytes from its
                            tensor's base (table entries at vector starts are multiples of 16 or 4 bytes; 16 also says
                            that no tile is moved back along a vector direction); else 0.  The kernels that load
-                           their operand tiles straight into LDS take only such problems (most of them only 16), and
-                           only when the base addresses are aligned likewise (checked at the launch, which
-                           otherwise runs the class's largest register-staged tile instead)  */
+                           their operand tiles straight into LDS take only such problems (most of them only 16; 1 counts as
+                           16), and only when the base addresses are aligned likewise (checked at the launch, which
+                           otherwise runs the register-staged tile named below instead)  */
     int32_t x_max_off, y_max_off; /* largest element offset xp[p] + xk[k] (yq[q] + yk[k]) over p < P, k < K:
                                      the kernels that build load addresses from table entries they have
                                      themselves moved through LDS clamp every address to it, and the
@@ -119,6 +121,10 @@ typedef struct hiptk_problem
                                      xk[k] == x_vec).  The kernels that load operand tiles straight into LDS and
                                      read k offsets from the tables then stage the operand chunk-major, so that
                                      neighbouring lanes load neighbouring memory.  Any value gives the same results */
+    int32_t unaligned_tile, unaligned_split; /* what runs in the tile's place where an operand's base is not aligned for it: a
+                                     register-staged tile of the class, in so many slices or as many of them as the
+                                     workspace of the call holds.  unaligned_split 0: not said, the class's largest
+                                     register-staged tile in split_k slices                                    */
     /* Filled by hiptk_resolve (zero otherwise): the registry entries this problem runs, looked up once
      * when the plan is made instead of at every launch.  `kernel` is what hiptk_kernel_name names;
      * `kernel_unaligned` is what runs in its place when X or Y is not aligned for it at the launch (the
@@ -141,7 +147,7 @@ const char* hiptk_kernel_name(const hiptk_problem_t* prob);
  * none.  Optional: hiptk_contract searches when the two fields are null. */
 int hiptk_resolve(hiptk_problem_t* prob);
 /* Name of the kernel a launch with these operand addresses runs: the resolved (or looked-up) kernel,
- * or its register-staged stand-in when X or Y is not 16-byte aligned. */
+ * or its register-staged stand-in when X or Y is not aligned for it. */
 const char* hiptk_kernel_name_at(const hiptk_problem_t* prob, const void* X, const void* Y);
 
 /* Bytes of workspace the problem needs (0 when split_k == 1). */
