@@ -326,6 +326,16 @@ namespace hipta
         };
         out.mode_i2 = out.mode_j2 = -1;
         out.chunk_i = out.chunk_j = 1;
+        // Kernels that take A at any element, chosen for its layout where one that reads vectors would be allowed: A's alignment
+        // still has to be what those vectors ask (a move into a packed copy is planned for the declared alignment and refuses
+        // an operand below it, whichever kernel it runs).  `linear`: the vectors run along A's first two modes.
+        auto vectorsOfA = [&](bool linear) {
+            std::vector<int64_t> others;
+            for(int d = 1; d < r; ++d)
+                if(!linear || d != jB)
+                    others.push_back(as[d]);
+            return in.elem_bytes * pickVec(in.elem_bytes, cap, linear ? ext[0] * ext[jB] : ext[0], others, in.A, false);
+        };
         int        kernel;
         if(tune.kernel == HIPTK_PERM_GROUPED && (tryGrouped(true, true) || tryShared(true)))
             return PermuteStatus::OK;
@@ -354,9 +364,15 @@ namespace hipta
             // 57 x 749 in strips 13.7 and 2.4.  (Extents that the small tiles cover to the last lane: 3.5-3.6 us in those.)
             kernel = HIPTK_PERM_GATHER;
         else if(smallStrip && in.elem_bytes == 4)
-            kernel = HIPTK_PERM_TILED;
+        {
+            kernel      = HIPTK_PERM_TILED;
+            out.a_align = vectorsOfA(stripI);
+        }
         else if(smallStrip && tryGrouped(true, false))
+        {
+            out.a_align = vectorsOfA(stripI);
             return PermuteStatus::OK;
+        }
         else if((stripJ && ext[0] >= 64) || (stripI && ext[jB] >= 64))
             kernel = HIPTK_PERM_STRIP;
         else if(shared && tune.tile < 0 && tryShared(false))
@@ -365,9 +381,13 @@ namespace hipta
             kernel = ext[0] >= 16 ? HIPTK_PERM_ROWS : HIPTK_PERM_GATHER;
         // (the plain tiles need 16 and more; and up to 2^23 f16 they make too few workgroups, where grouped ones are cut
         // until they make enough: 692 x 464 10.1 us in tiles, 4.2 grouped, 691 x 4279 11.8 and 7.2, 123 x 40061 11.1 and 10.2)
-        else if(tune.tile < 0
-                && tryGrouped(ext[0] < 16 || ext[jB] < 16 || (tune.kernel < 0 && in.elem_bytes == 2 && count <= (1 << 23) && (count >= (1 << 18) || !whole)), false))
+        else if(tune.tile < 0 && tryGrouped(ext[0] < 16 || ext[jB] < 16, false))
             return PermuteStatus::OK;
+        else if(tune.tile < 0 && tune.kernel < 0 && in.elem_bytes == 2 && count <= (1 << 23) && (count >= (1 << 18) || !whole) && tryGrouped(true, false))
+        {
+            out.a_align = vectorsOfA(false);
+            return PermuteStatus::OK;
+        }
         else
         {
             kernel = (ext[0] >= 16 && ext[jB] >= 16) ? HIPTK_PERM_TILED : HIPTK_PERM_GATHER;
@@ -376,8 +396,11 @@ namespace hipta
             const int    order[] = {0, 1, 2};
             const Tile   t       = (in.elem_bytes == 4 ? TILES4 : TILES2)[pickTile(in.elem_bytes, ext[0], ext[jB], order)];
             const double inside  = coverage(ext[0], t.ti) * coverage(ext[jB], t.tj);
-            if(tune.kernel < 0 && tune.tile < 0 && inside < 0.15)
-                kernel = HIPTK_PERM_GATHER;
+            if(tune.kernel < 0 && tune.tile < 0 && inside < 0.15 && kernel == HIPTK_PERM_TILED)
+            {
+                kernel      = HIPTK_PERM_GATHER;
+                out.a_align = vectorsOfA(false);
+            }
         }
         out.kernel = kernel;
         if(kernel == HIPTK_PERM_GATHER)
@@ -456,7 +479,8 @@ namespace hipta
             if(const int er = pickVec(in.elem_bytes, full, ext[0], aOthers, nullptr, false), ew = pickVec(in.elem_bytes, full, ext[jB], bOthers, nullptr, false);
                tune.loose || (cap >= full && tune.kernel < 0 && (in.elem_bytes == 2 ? std::min(er, ew) == 1 : er < full)))
             {
-                out.loose = 1;
+                out.loose   = 1;
+                out.a_align = std::max(out.a_align, out.vec_r * in.elem_bytes);
                 out.vec_r = out.vec_w = full;
             }
         }

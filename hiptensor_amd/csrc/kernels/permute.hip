@@ -1075,7 +1075,7 @@ extern "C" int hiptk_permute(const hiptk_permute_t* p, const void* A, void* B, v
     int64_t n = 0;
     if(!well_formed(p, &n) || !A || !B)
         return HIPTK_ERR_ARG;
-    if(!aligned(A, p->elem_bytes) || !aligned(B, p->elem_bytes))
+    if(!aligned(A, p->elem_bytes) || !aligned(B, p->elem_bytes) || (p->a_align > 1 && !aligned(A, p->a_align)))
         return HIPTK_ERR_ARG;
     hipStream_t s  = static_cast<hipStream_t>(stream);
     int         rc = -1;

@@ -248,6 +248,8 @@ typedef struct hiptk_permute
     int32_t width_i, width_j; /* GROUPED: elements of mode 0 / mode_j per tile                    */
     int32_t loose; /* GROUPED, TILED: 16-byte vectors that start at any element and need divide nothing
                       (vec_r == vec_w == 16 / elem_bytes)                                         */
+    int32_t a_align; /* bytes that A must start at a multiple of beside what vec_r asks (0: nothing): a move planned
+                        for an operand of a declared alignment refuses one below it with every kernel  */
     int32_t bands; /* TILED / GROUPED: 1: each die takes neighbouring tiles                       */
     int32_t keep;  /* TILED / GROUPED: 1: B is written with ordinary stores instead of non-temporal ones (runs of
                       B that start inside a line: two tiles write parts of it)                    */
