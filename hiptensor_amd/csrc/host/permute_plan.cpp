@@ -475,9 +475,15 @@ namespace hipta
             // line moved back to end with it), for single f16 and for f32 that is read in less (f16 2712 x 81993 230 -> 218
             // us, 1943.205.637 -> (2,1,0) 460 -> 261, 4459 x 2670 26.0 -> 18.1; f32 2073.32.279 -> (2,1,0) 42.9 -> 37.6).  Not
             // for pairs of f16 (324.350.368 -> (1,2,0) 49 -> 61) nor f32 read whole (164.329.609 -> (1,0,2) 62.8 -> 66.7).
+            // Of f16 with pairs on one side and single elements on the other not those written in pairs from the tile of 32
+            // columns (75 random shapes 1.25 of the time up to 2^25 elements, 1.49 beyond), nor large matrices with columns of 3000
+            // and more read in pairs on tiles of 128 columns (258: 1.07, 178 of them above 1.05) or written in pairs from 128 x 128
+            // (38: 1.22); with shorter columns, more modes or fewer elements those take 0.79-0.97, the others 0.61-0.95.
             // (Narrow for the extents' sake: a base off its alignment alone keeps the vectors it admits.)
-            if(const int er = pickVec(in.elem_bytes, full, ext[0], aOthers, nullptr, false), ew = pickVec(in.elem_bytes, full, ext[jB], bOthers, nullptr, false);
-               tune.loose || (cap >= full && tune.kernel < 0 && (in.elem_bytes == 2 ? std::min(er, ew) == 1 : er < full)))
+            const int  er = pickVec(in.elem_bytes, full, ext[0], aOthers, nullptr, false), ew = pickVec(in.elem_bytes, full, ext[jB], bOthers, nullptr, false);
+            const bool large  = r == 2 && count > (1 << 25) && ext[jB] >= 3000, square = out.tile == 0;
+            const bool single = std::min(er, ew) == 1 && !(ew == 2 && (out.tile == 1 || (large && square))) && !(er == 2 && large && (square || out.tile == 3));
+            if(tune.loose || (cap >= full && tune.kernel < 0 && (in.elem_bytes == 2 ? single : er < full)))
             {
                 out.loose   = 1;
                 out.a_align = std::max(out.a_align, out.vec_r * in.elem_bytes);
