@@ -565,15 +565,21 @@ namespace hipta
         for(int d = 0; d < out.rank; ++d)
             if(d != jB && out.b_stride[d] * (int64_t)out.elem_bytes % 64 != 0)
                 runs64 = 0;
-        // (blocks transposed in place share no line with another tile's block that ordinary stores could put together: f16
-        // 96.78.191.51 -> (1,0,2,3) 55 us, 63 with both)
-        const bool inPlace = out.rank >= 2 && jB == 1 && out.b_stride[0] == out.extent[1];
-        if(inPlace)
-            return PermuteStatus::OK;
-        const Tile* ts = out.elem_bytes == 4 ? TILES4 : TILES2;
+        // (a matrix, or blocks, transposed in place)
+        const bool  inPlace = out.rank >= 2 && jB == 1 && out.b_stride[0] == out.extent[1];
+        const Tile* ts      = out.elem_bytes == 4 ? TILES4 : TILES2;
         switch(out.kernel)
         {
         case HIPTK_PERM_TILED:
+            // In place the order of the tiles decides less where no two tiles write parts of one line: blocks that one tile holds
+            // (f32 36.35.2423 -> (1,0,2) 9.9 us, 11.0 with both), runs of whole 64 bytes in vectors that divide them (44 shapes of
+            // 2^24 elements and more 1.03 of the time, up to 1.11) and the f16 tile of 512 columns (1.02, up to 1.26).  Elsewhere
+            // sixteen tiles along j without a die to share them lose against one tile (f16 342.799.566 -> (1,0,2) 182 -> 233 us, 1848 x
+            // 117198 214 -> 276; with both 130 and 204: 415 shapes 0.81 of the time).
+            if(inPlace
+               && ((out.extent[0] <= ts[out.tile].ti && out.extent[jB] <= ts[out.tile].tj) || (runs64 && !out.loose)
+                   || (out.elem_bytes == 2 && ts[out.tile].ti < 64)))
+                break;
             // neighbours on one die also share what they read: 46 random shapes 0.92 of the time, aligned ones among them
             // (f32 1 GiB 379.5 -> 371).  Ordinary stores where the runs are shorter than lines, and on tensors the caches
             // do not hold (up to there they cost 5-10 %: f32 3607 x 590 7.8 -> 8.5, 2307 x 2322 11.8 -> 12.9).
@@ -585,6 +591,9 @@ namespace hipta
         case HIPTK_PERM_GROUPED:
             // 30 random shapes 0.91 of the time on neighbouring tiles (f32 8.57.15.7.55.66 -> (5,4,2,3,1,0) 490 -> 323, 1.02
             // at the worst), 0.90 with ordinary stores besides
+            // (not in place, where such blocks share no line: f16 96.78.191.51 -> (1,0,2,3) 55 us, 63 with both)
+            if(inPlace)
+                break;
             out.bands = 1;
             out.keep  = !runs64;
             break;

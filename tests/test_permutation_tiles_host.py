@@ -37,3 +37,13 @@ def test_choice(host_handle, dtype, lens, perm, name):
     got = p.info(0, 0)["kernel_name"]
     p.close()
     assert got == name
+
+
+def test_tiles_that_share_lines_go_to_one_die(tmp_path):
+    """tests/cpp/tile_order.cpp: matrices and blocks transposed in place, and others, with the tile order of their plan."""
+    src, out = os.path.join(ROOT, "tests", "cpp", "tile_order.cpp"), tmp_path / "tile_order"
+    subprocess.run(["g++", "-std=c++17", "-O1", "-I" + os.path.join(ROOT, "include"), "-isystem", "/opt/rocm/include",
+                    "-D__HIP_PLATFORM_AMD__", src, "-o", str(out), "-L" + os.path.dirname(_lib.LIB_PATH), "-lhiptensor_amd",
+                    "-Wl,-rpath," + os.path.dirname(_lib.LIB_PATH)], check=True, capture_output=True)
+    r = subprocess.run([str(out)], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0 and r.stdout.strip().splitlines()[-1].startswith("ok"), (r.stdout[-2000:], r.stderr)
