@@ -397,8 +397,11 @@ namespace hipta
     {
         if(c.sol->vec_align == 0)
             return nullptr;
+        // The 32/64-bit 64 x 64 tiles add in the order of the staged tiles: in the same slices, so that a result does not depend on
+        // where the operands lie.  (16-bit tiles add in another order, the 32 x 32 tiles' waves split K.)
+        const bool same_bits = class_flops_per_clk_cu(c.sol->cls) != 4096.0 && c.sol->bp * c.sol->bq >= 4096;
         for(const Choice& o : ranked)
-            if(o.sol->vec_align == 0)
+            if(o.sol->vec_align == 0 && (!same_bits || o.split_k == c.split_k))
                 return &o;
         return nullptr;
     }

@@ -72,7 +72,7 @@ namespace hipta
                                      const DeviceModel&                  dev);
 
     // What runs where an operand's base is not aligned for `c`: the best register-staged choice of the ranking that `c`
-    // comes from (nullptr: `c` takes any base, or there is none).
+    // comes from, of those that give the same bits if any can (nullptr: `c` takes any base, or there is none).
     const Choice* stand_in(const Choice& c, const std::vector<Choice>& ranked);
 
     // MFMA flop per clock per CU of a class (dense peak), for estimates and reports.

@@ -77,9 +77,11 @@ int main()
                 CHECK(o, "%s: nothing to stand in", name);
                 if(!o)
                     continue;
-                // the best staged choice there is
+                // the best staged choice there is, in the same slices where the tiles add in the same order
+                const bool same_bits = v.cls != HIPTK_F16 && v.cls != HIPTK_BF16 && c.sol->bp == 64;
+                CHECK(!same_bits || o->split_k == c.split_k, "%s: stand-in in %d", name, o->split_k);
                 for(const Choice& s : ranked)
-                    CHECK(s.sol->direct || o->est_us <= s.est_us, "%s: %s in %d beats the stand-in", name, s.sol->name.c_str(), s.split_k);
+                    CHECK(s.sol->direct || (same_bits && s.split_k != c.split_k) || o->est_us <= s.est_us, "%s: %s in %d beats the stand-in", name, s.sol->name.c_str(), s.split_k);
                 hiptk_problem_t p{};
                 p.cls = v.cls, p.tile_id = c.sol->tile_id, p.split_k = c.split_k, p.P = v.P, p.Q = v.Q, p.K = v.K;
                 p.x_kfast = v.x_kfast, p.y_kfast = v.y_kfast, p.x_vec = v.x_vec, p.y_vec = v.y_vec, p.k_affine = v.k_affine;
