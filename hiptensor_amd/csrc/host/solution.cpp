@@ -332,10 +332,11 @@ namespace hipta
         // the fabric (256 x 256 x 65536 f16 in 32 slices: 16 tiles of 64 x 64 move 2.7e8 B for 6.7e7 algorithmic
         // and take 40.5 us, 4 tiles of 128 x 128 move half of that and take 33.4)
         // (a little more of them where an XCD takes whole slices, whose tiles then meet in its L2: launch.hip; f64 110 x 324 x
-        // 112500 on 32 x 32 tiles in 16 slices 231 us, on 64 x 64 in 64 190)
-        const bool slice_bands = split >= 8 && std::ceil(ktiles / split) * split >= 160;
+        // 112500 on 32 x 32 tiles in 16 slices 231 us, on 64 x 64 in 64 190.  With 1.4 there too the tiles chosen are larger, 0.80-0.93 of the
+        // time with operands of 200 MB and more, but the slices fewer: 54 random contractions 1.00, 16 of them above 1.05)
         if(split > 1)
-            us = std::max(us, tiles * (double)(s.bp + s.bq) * (double)v.K * v.elem_bytes / (dev.hbm_gbs * 1e3 * (slice_bands ? 1.75 : 1.4)));
+            us = std::max(us, tiles * (double)(s.bp + s.bq) * (double)v.K * v.elem_bytes
+                                  / (dev.hbm_gbs * 1e3 * (hiptk_slices_by_die((int64_t)ktiles, split) ? 1.75 : 1.4)));
         // launch, and prologue + epilogue of every round of workgroups on a CU
         // (a workgroup's epilogue moves its output tile, and C, at about 30 GB/s per CU)
         const double tile_io = (double)s.bp * s.bq * v.elem_bytes * (v.bilinear ? 2.0 : 1.0) / 30e3;

@@ -512,6 +512,20 @@ extern "C" uint64_t hiptk_workspace_bytes(const hiptk_problem_t* prob)
            * (uint64_t)hiptk::acc_bytes(prob->cls);
 }
 
+// Many long slices: an XCD takes whole slices, whose tiles read the same panels, instead of a band of every
+// slice's tiles, where each panel went to all eight L2s (bf16 324 x 207 x 52974 in 32 slices 40.8 -> 23.4 us, f64
+// 116 x 144 x 54844 in 16 87.0 -> 66.8, f32 256 x 256 x 65536 in 32 76.5 -> 71.8).  Few or short slices start on
+// cold panels all at once, and the tiles of one wait on the same lines: 1.00-1.11 of the time (c32 320 x 768 x 128
+// in 4 11.2 -> 12.4, bf16 1024 x 224 x 800 in 8 18.7 -> 19.4).
+extern "C" int hiptk_slices_by_die(int64_t ktiles, int64_t split)
+{
+    if(ktiles < 1 || split < 1)
+        return 0;
+    const int64_t per    = (ktiles + split - 1) / split;
+    const int64_t slices = (ktiles + per - 1) / per;
+    return slices >= 8 && slices * per >= 160;
+}
+
 extern "C" int hiptk_contract(const hiptk_problem_t* prob,
                               const void*            alpha,
                               const void*            beta,
@@ -602,13 +616,7 @@ extern "C" int hiptk_contract(const hiptk_problem_t* prob,
     a.ktiles_per_split = (ktiles + split - 1) / split;
     split              = (ktiles + a.ktiles_per_split - 1) / a.ktiles_per_split; // no empty slice
     a.split_k          = split;
-    // Many long slices: an XCD takes whole slices, whose tiles read the same panels, instead of a band of every
-    // slice's tiles, where each panel went to all eight L2s (bf16 324 x 207 x 52974 in 32 slices 40.8 -> 23.4 us, f64
-    // 116 x 144 x 54844 in 16 87.0 -> 66.8, f32 256 x 256 x 65536 in 32 76.5 -> 71.8).  Few or short slices start on
-    // cold panels all at once, and the tiles of one wait on the same lines: 1.00-1.08 of the time (c32 320 x 768 x 128
-    // in 4 11.2 -> 12.4, bf16 1024 x 224 x 800 in 8 18.7 -> 19.4).
-    a.slice_bands = split >= 8 && (int64_t)split * a.ktiles_per_split >= 160
-                            && (uint64_t)a.tiles_p * (uint64_t)a.tiles_q * (uint64_t)split <= 0x7FFFFFFFull
+    a.slice_bands = hiptk_slices_by_die(ktiles, split) && (uint64_t)a.tiles_p * (uint64_t)a.tiles_q * (uint64_t)split <= 0x7FFFFFFFull
                         ? 1
                         : 0;
     if((uint64_t)a.tiles_p * (uint64_t)a.tiles_q > 0x7FFFFFFFull || split > 65535)

@@ -150,6 +150,10 @@ int hiptk_resolve(hiptk_problem_t* prob);
  * or its register-staged stand-in when X or Y is not aligned for it. */
 const char* hiptk_kernel_name_at(const hiptk_problem_t* prob, const void* X, const void* Y);
 
+/* A launch over `ktiles` K tiles in at most `split` slices: 1 if it deals whole slices to the dies, 0 if it deals every slice's
+ * tiles.  What the launch does and what its estimate goes by. */
+int hiptk_slices_by_die(int64_t ktiles, int64_t split);
+
 /* Bytes of workspace the problem needs (0 when split_k == 1). */
 uint64_t hiptk_workspace_bytes(const hiptk_problem_t* prob);
 
