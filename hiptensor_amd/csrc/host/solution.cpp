@@ -328,6 +328,11 @@ namespace hipta
             // rates say: 901 x 176 x 332 c32 11.0 and 25.1)
             us = std::max(us, bytes / (dev.hbm_gbs * 1e3 * (any_split_lines && s.bp * s.bq < 4096 ? 0.32 : 0.6)));
         }
+        // ... and slices of one row of their 64 x 64 tiles, with operands the last-level cache does not keep, read the tiles' panels at
+        // 3.1-4.0 TB/s: f64 5487 x 55 x 5035 in eight 121 us, staged in eight 88; 9000 x 46 x 1733 in four 72 and 58 (a small side of 4 to
+        // 15: 39-42, staged 45-51)
+        if(any_split_lines && split > 1 && s.bp * s.bq >= 4096 && std::min(v.P, v.Q) <= 64 && bytes > 110e6)
+            us = std::max(us, tiles * (double)(std::min<int64_t>(s.bp, v.P) + std::min<int64_t>(s.bq, v.Q)) * (double)v.K * v.elem_bytes / (dev.hbm_gbs * 1e3 * 0.42));
         // split-K slices of different tiles share nothing in time: every workgroup's operand panels come through
         // the fabric (256 x 256 x 65536 f16 in 32 slices: 16 tiles of 64 x 64 move 2.7e8 B for 6.7e7 algorithmic
         // and take 40.5 us, 4 tiles of 128 x 128 move half of that and take 33.4)
