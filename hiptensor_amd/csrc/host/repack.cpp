@@ -101,7 +101,10 @@ namespace hipta
             // read once, written once, plus a launch.  Measured on operands of 10-20 MB with runs of
             // 15 elements: the element-wise fallback moves 1.2 (2-byte) to 2.0 TB/s (4-byte), the
             // tile kernels 1.6-3.2 TB/s (5-6 TB/s on large tensors with long runs)
-            const double rate = po.perm.kernel == HIPTK_PERM_GATHER ? (pin.elem_bytes == 2 ? 1.2e6 : 2.0e6) : 2.5e6; // bytes / us
+            // (shared tiles of a few elements, which the workgroups are started for one by one: c32 3.4.3.27336 in tiles of 3 x 3 135 us
+            // for 7.9 MB)
+            const bool   tiny = po.perm.kernel == HIPTK_PERM_SHARED && po.perm.extent[0] * po.perm.chunk_i * po.perm.chunk_j < 64;
+            const double rate = po.perm.kernel == HIPTK_PERM_GATHER ? (pin.elem_bytes == 2 ? 1.2e6 : 2.0e6) : tiny ? 0.12e6 : 2.5e6; // bytes / us
             po.est_us         = 2.0 * raw / rate + 3.0;
 
             packed       = t;
@@ -164,29 +167,6 @@ namespace hipta
         }
     }
 
-    namespace
-    {
-        // A choice's estimate as it compares with a plan of another layout.  The cost of a split-K slice is set so that the
-        // best number of slices comes out first; for the tiles staged through registers in vectors it is above what the slices
-        // take (median over 125 drawn problems: 2 us with 2 to 4 slices, 3 with 8, 4 with 16, 7 with 32; element by element
-        // only with 64).
-        double comparable_us(const Choice& c, const GemmView& v)
-        {
-            return c.split_k > 1 && !c.sol->direct && (std::min(v.x_vec, v.y_vec) > 1 || c.split_k >= 64) ? c.est_us - std::min(6.0, 1.5 + 0.16 * c.split_k) : c.est_us;
-        }
-
-        // ... of a plan on packed copies.  (8-byte elements: without the tiles that take operands at any element, which a copy of odd
-        // extents would run.  The element-by-element gather it saves there is within 13 % of whole vectors, less than the estimates
-        // of the moves and of those tiles are good for.)
-        double packed_us(const std::vector<Choice>& ranked, const GemmView& v)
-        {
-            for(const Choice& c : ranked)
-                if(!(v.elem_bytes == 8 && c.sol->direct && c.sol->tile_id >= 4))
-                    return comparable_us(c, v);
-            return comparable_us(ranked.front(), v);
-        }
-    }
-
     RepackMode repack_mode_from_env()
     {
         const char* e = std::getenv("HIPTENSOR_AMD_REPACK");
@@ -223,7 +203,7 @@ namespace hipta
         if(!ma.eligible && !mb.eligible)
             return PlanStatus::OK;
         const int    es        = out.view.elem_bytes;
-        const double base_us   = comparable_us(out.ranked.front(), out.view);
+        const double base_us   = expected_us(out.ranked.front(), out.view);
         double       best_us   = 0.0;
         bool         have_best = false;
         ContractionPlanChoice best;
@@ -266,7 +246,14 @@ namespace hipta
                 alt.ranked = rank_choices(candidates, alt.view, std::min(max_ws - alt.pack_bytes, split_cap), dev);
                 if(alt.ranked.empty())
                     continue;
-                double us = packed_us(alt.ranked, alt.view) + alt.a.est_us + alt.b.est_us;
+                double us = expected_us(alt.ranked.front(), alt.view) + alt.a.est_us + alt.b.est_us;
+                // (1 036 random contractions an operand of which has no whole vectors, each planned without copies and with each pair of
+                // them: the choice takes 0.987 of the time of packing as it was decided before direct-load tiles of ordinary size, 13
+                // above 1.05.  0.9 of the estimates instead, with or without their correction for slices: 0.990-0.993, 18 to 31.  Two
+                // copies of 8-byte elements, which the element-by-element gather reads within 13 % of whole vectors, have to promise
+                // more: 4845 x 4845 x 1001 in copies 0.83-0.94 of the time in place, 1500 x 1500 x 1001 0.92-1.06)
+                if(mode != RepackMode::FORCE && us >= (es == 8 && alt.a.on && alt.b.on ? 0.84 * base_us : base_us - 1.0))
+                    continue;
                 if(mode == RepackMode::FORCE)
                     us -= 1e9 * ((alt.a.on ? 1 : 0) + (alt.b.on ? 1 : 0)); // as many copies as the layouts admit
                 if(!have_best || us < best_us)
@@ -276,8 +263,7 @@ namespace hipta
                     have_best = true;
                 }
             }
-        // a packed plan has to promise a clear gain: the estimates are good to about ten percent
-        if(have_best && (mode == RepackMode::FORCE || best_us < 0.9 * base_us))
+        if(have_best)
             out = std::move(best);
         return PlanStatus::OK;
     }

@@ -399,6 +399,18 @@ namespace hipta
         return out;
     }
 
+    double expected_us(const Choice& c, const GemmView& v)
+    {
+        // The cost of a split-K slice in estimate_us is set so that the best number of slices comes out first.  For the tiles staged
+        // through registers that is above what the slices take: over 276 random contractions of up to 25 us by a median of 1.3 us
+        // in 2 to 4 slices, 2.9 in 8, 4.8 in 16, 6.4 in 32 and 9.3 in 64 (16-bit elements one by one of one operand more, of both and
+        // 32-bit ones less); a little over half of it decides best (repack.cpp).
+        if(c.split_k <= 1 || c.sol->direct)
+            return c.est_us;
+        const bool narrow = std::min(v.x_vec, v.y_vec) * v.elem_bytes < 8;
+        return c.est_us - (!narrow ? 0.75 : v.elem_bytes == 2 && std::max(v.x_vec, v.y_vec) > 1 ? 1.0 : 0.5) * (std::log2((double)c.split_k) - 1.0);
+    }
+
     const Choice* stand_in(const Choice& c, const std::vector<Choice>& ranked)
     {
         if(c.sol->vec_align == 0)

@@ -71,6 +71,9 @@ namespace hipta
                                      uint64_t                            max_ws,
                                      const DeviceModel&                  dev);
 
+    // What a choice's estimate comes to, where it is compared with a plan of another layout.
+    double expected_us(const Choice& c, const GemmView& v);
+
     // What runs where an operand's base is not aligned for `c`: the best register-staged choice of the ranking that `c`
     // comes from, of those that give the same bits if any can (nullptr: `c` takes any base, or there is none).
     const Choice* stand_in(const Choice& c, const std::vector<Choice>& ranked);
