@@ -45,6 +45,7 @@ namespace hiptk
         static constexpr int LDS_BYTES = NS * STAGE * 2;
         static_assert(TP >= 1 && TQ >= 1 && BP % (WP * 32) == 0 && BQ % (WQ * 32) == 0, "whole wave tiles");
         static_assert(NS >= 2 && (NS - 2) * LPT < 64, "the wait counts must fit vmcnt");
+        static_assert(NS <= 4, "last_steps tells up to two tiles on their way apart");
         static_assert(LDS_BYTES <= 160 * 1024 && LDS_BYTES >= 4 * 32 * (TQ * 32 + 4) * 4, "LDS of one CU; the epilogue's staging");
     };
 
@@ -134,7 +135,7 @@ namespace hiptk
                 const int k = 8 * (lane >> 4) + ((lane & 15) >> 2);
 #pragma unroll
                 for(int b = 0; b < NB; b++)
-                    frag[b] = k * BR + hm_row_pos<BR>(wrow + 16 * b + 4 * (lane & 3), k);
+                    frag[b] = k * BR + hd_row_pos(wrow + 16 * b + 4 * (lane & 3), k);
             }
         }
         __device__ inline u32x4_t fetch(const uint16_t* stage, int b, int ks) const
@@ -251,8 +252,6 @@ namespace hiptk
             const bool more   = t + NS < sl.nt;
             if(behind >= NS - 2)
                 step(std::integral_constant<int, NS - 2>{}, more, cur, nxt);
-            else if(NS > 4 && behind == 2)
-                step(std::integral_constant<int, 2>{}, false, cur, nxt);
             else if(NS > 3 && behind == 1)
                 step(std::integral_constant<int, 1>{}, false, cur, nxt);
             else if(behind == 0)

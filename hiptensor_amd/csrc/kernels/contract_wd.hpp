@@ -32,9 +32,10 @@
 //     1920 x 1920 x 768 f64 took 107.7 us, without them 100.5, without the test 98.0.
 //
 // Restrictions (the dispatcher checks them): both operands gathered in 16-byte vectors, along their
-// row index or along k, on 16-byte boundaries; one K stride per operand; K at least BK (a last tile
-// shorter than BK loads the vectors beyond K from zeros), and a multiple of the vector where an operand
-// is contiguous along k; byte offsets inside each operand below 2^32.
+// row index or along k; one K stride per operand; K at least BK (a last tile shorter than BK loads the vectors
+// beyond K from zeros); byte offsets inside each operand below 2^32.  contract_wd_kernel: vectors on 16-byte
+// boundaries, K a multiple of the vector where an operand is contiguous along k, no tile moved back.
+// contract_wx_kernel: vectors at any element, any K, the last tile of rows that are one ragged run moved back.
 #pragma once
 #include <utility>
 
@@ -108,8 +109,9 @@ namespace hiptk
     // contract_w.hpp's epilogue_w fetches four accumulator rows at a time behind the stores of the four
     // before (D may alias C), one memory latency per batch, which other workgroups on the CU cover there;
     // here a workgroup may be alone, and the registers for all of a lane's C elements are free.
-    // (Reading C early is safe when D aliases it: every element is read and written by the same lane,
-    // these kernels never move a tile back over a neighbour's rows.)
+    // (Reading C early is safe when D aliases it: an element is read for its value and written by one lane only, that of
+    // the tile which owns it.  A tile that is moved back over its neighbour's rows (contract_wx_kernel) neither uses C
+    // nor stores there: `pmask` and `qmask` hold its own rows and columns.)
     template <typename Tr, int TP, int TQ>
     struct WdEpilogue
     {

@@ -206,8 +206,8 @@ namespace hiptk
 
     // ---- 16-bit kernel for tiles smaller than 256 (contract_hm.hpp): K tiles of 64, stages as above ----
     // The K tiles one workgroup reduces, in the order it takes them: when the slice ends at K and K is not a
-    // multiple of 64, the tile with the last tail_k k comes first (its loads are the ones that need tests and may be
-    // more than a whole tile's, which the waits for any later tile then need not count), then the whole tiles.
+    // multiple of 64, the tile with the last tail_k k comes first (its loads are the ones that need tests, and no step of
+    // the main loop has to look for it; it takes as many of them as a whole tile), then the whole tiles.
     struct HmSlice
     {
         int nt, tail_k, k00;
@@ -227,14 +227,8 @@ namespace hiptk
     {
         return s.tail_k == 0 ? s.k00 + u * HK_BK : u == 0 ? s.k00 + (s.nt - 1) * HK_BK : s.k00 + (u - 1) * HK_BK;
     }
-    // chunks of 8 rows are exchanged within a k-row so that the four k-rows a transposing read of 16 lanes touches lie
-    // in different banks; 32 rows are 64 bytes, four of which are in different banks as they are
-    template <int BR>
-    HIPTK_HD_FN int hm_row_pos(int row, int k)
-    {
-        return BR >= 64 ? hd_row_pos(row, k) : row;
-    }
-    // what the 16-byte slot s of a stage holds
+    // what the 16-byte slot s of a stage holds (row-contiguous: chunks of 8 rows are exchanged within a k-row, hd_row_pos, so that
+    // the four k-rows a transposing read of 16 lanes touches lie in different banks)
     template <bool KF, int BR>
     HIPTK_HD_FN HdSlot hm_slot(int s)
     {
@@ -243,7 +237,8 @@ namespace hiptk
         HdSlot        o;
         constexpr int cpr = BR / 8;
         o.k               = s / cpr;
-        o.row             = hm_row_pos<BR>(8 * (s % cpr), o.k);
+        static_assert(BR >= 64, "hd_row_pos exchanges eight chunks");
+        o.row = hd_row_pos(8 * (s % cpr), o.k);
         return o;
     }
     // The k (from the tile's origin, so -6 .. 63) that is loaded at k-position k of the tile of which only tail_k k lie

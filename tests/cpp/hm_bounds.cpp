@@ -90,7 +90,7 @@ static void walk_operand(const char* name, const Operand& o, int r0, const HmSli
                     {
                         const int r = s.row + (KF ? 0 : j), pos = s.k + (KF ? j : 0);
                         // where the operand fetch looks for (r, pos)
-                        const int want = KF ? r * HK_BK + 8 * hk_chunk_pos(r, pos / 8) + pos % 8 : pos * BR + hm_row_pos<BR>(r, pos);
+                        const int want = KF ? r * HK_BK + 8 * hk_chunk_pos(r, pos / 8) + pos % 8 : pos * BR + hd_row_pos(r, pos);
                         CHECK(want == 8 * q + j, "%s (%d, %d) lands at %d, is read at %d", name, r, pos, 8 * q + j, want);
                         seen[(size_t)(r * HK_BK + pos)]++;
                         const int64_t source = source_k(K, ko, pos, chunks);
@@ -111,7 +111,7 @@ static void walk_operand(const char* name, const Operand& o, int r0, const HmSli
         // a transposing read takes 4 rows at one k in one go
         for(int r = 0; !KF && r < BR; r += 4)
             for(int k = 0; k < 8; k++)
-                CHECK(hm_row_pos<BR>(r + 3, k) == hm_row_pos<BR>(r, k) + 3 && hm_row_pos<BR>(r, k) % 4 == 0, "%s rows %d.. at k %d", name, r, k);
+                CHECK(hd_row_pos(r + 3, k) == hd_row_pos(r, k) + 3 && hd_row_pos(r, k) % 4 == 0, "%s rows %d.. at k %d", name, r, k);
     }
 }
 
