@@ -63,7 +63,7 @@ struct Case
     std::vector<int32_t>                     mA, mB, mD; // modes as listed
     std::vector<std::pair<int32_t, int64_t>> ext;
     std::vector<int32_t>                     oA, oB, oD; // storage order, fastest first (empty: as listed)
-    int64_t                                  padD = 0; // elements added after D's fastest mode
+    int64_t                                  padD = 0, padAB = 0; // elements added after D's (A's and B's) fastest mode
     bool                                     bilinear = false;
 };
 
@@ -655,13 +655,26 @@ int main()
             cases.push_back(c);
         }
     }
+    // vectors at multiples of 4 bytes, not 16: rows (or k-rows) of two f16 elements beyond a multiple of eight
+    for(const char* form : {"rowfast", "kfast", "mixed"})
+    {
+        Case c;
+        c.name  = std::string("pad2_") + form;
+        c.ext   = {{0, 384}, {10, 320}, {20, 208}};
+        const bool akf = form[0] == 'k', bkf = form[0] != 'r';
+        c.mA = akf ? std::vector<int32_t>{20, 0} : std::vector<int32_t>{0, 20};
+        c.mB = bkf ? std::vector<int32_t>{20, 10} : std::vector<int32_t>{10, 20};
+        c.mD = {0, 10}, c.padAB = 2;
+        cases.push_back(c);
+    }
     long walked = 0;
+    int  at_4_bytes = 0;
     int  offered = 0, offered_hk = 0, offered_ring = 0, offered_ring_chunked = 0, computed_rows = 0;
     for(const Case& c : cases)
     {
         ProblemIn in;
-        in.A = tensor(c, c.mA, c.oA, 0);
-        in.B = tensor(c, c.mB, c.oB, 0);
+        in.A = tensor(c, c.mA, c.oA, c.padAB);
+        in.B = tensor(c, c.mB, c.oB, c.padAB);
         in.D = tensor(c, c.mD, c.oD, c.padD);
         in.bilinear = c.bilinear;
         if(c.bilinear)
@@ -673,6 +686,7 @@ int main()
         CHECK(st == PlanStatus::OK, "%s: %s", c.name.c_str(), why.c_str());
         if(st != PlanStatus::OK)
             continue;
+        at_4_bytes += v.xy_aligned == 4;
         // is a direct-load tile offered for it?  (tile ids 9: 256 x 256, 10: 256 x 192; on 16 x 16 x 32 MFMAs: 11: 256 x 256 in
         // K tiles of 64, one k stride per operand; 12: 256 x 192 in K tiles of 32 through a ring of four stages, k offsets from tables)
         for(int tile : {9, 10, 11, 12})
@@ -688,7 +702,7 @@ int main()
                         v.xy_aligned, tile, avail ? "offered" : "not offered");
             if(!avail)
                 continue;
-            CHECK(v.x_vec == 8 && v.y_vec == 8 && v.K % 16 == 0 && v.K >= 32 && v.xy_aligned, "%s offered outside its restrictions", c.name.c_str());
+            CHECK(v.x_vec == 8 && v.y_vec == 8 && v.K % 16 == 0 && v.K >= 32 && v.xy_aligned == 16, "%s offered outside its restrictions", c.name.c_str());
             if(tile == 11)
             {
                 computed_rows += check_computed_rows(c, v);
@@ -708,6 +722,7 @@ int main()
             walked += tile == 9 ? check_tile_size<256>(c, v) : check_tile_size<192>(c, v);
         }
     }
+    CHECK(at_4_bytes >= 3, "only %d cases with vectors at multiples of 4 bytes", at_4_bytes);
     CHECK(offered >= 40, "only %d (case, tile) pairs were offered a direct-load kernel", offered);
     CHECK(offered_hk >= 15, "only %d cases were offered the kernel with K tiles of 64", offered_hk);
     CHECK(computed_rows >= 10, "only %d cases of the K-tile-of-64 kernel have computed row offsets", computed_rows);
@@ -731,6 +746,17 @@ int main()
     rank4("k42_rowfast", {0, 1, 20, 21}, {10, 11, 20, 21}, {0, 1, 10, 11}, 40, 9, 24, 13, 6, 7);
     rank4("k42_kfast", {20, 21, 0, 1}, {20, 21, 10, 11}, {10, 11, 0, 1}, 40, 9, 24, 13, 6, 7);
     rank4("big_rowfast", {0, 1, 20, 21}, {10, 11, 20, 21}, {0, 1, 10, 11}, 8192, 16, 64, 1, 64, 64);
+    // vectors at multiples of 4 bytes, not 16 (complex f64, one element a vector, has none such)
+    for(int kf = 0; kf < 2; kf++)
+    {
+        Case c;
+        c.name = kf ? "pad1_kfast" : "pad1_rowfast";
+        c.ext  = {{0, 128}, {10, 192}, {20, 96}};
+        c.mA = kf ? std::vector<int32_t>{20, 0} : std::vector<int32_t>{0, 20}, c.mB = kf ? std::vector<int32_t>{20, 10} : std::vector<int32_t>{10, 20};
+        c.mD = {0, 10}, c.padAB = 1;
+        cases.push_back(c);
+    }
+    int            wide_at_4_bytes = 0;
     const WideTile wide[] = {{"f32", 0, 4, 4, 2, 16, 64}, {"f64", 1, 16, 8, 2, 8, 64}, {"c32", 4, 2048, 8, 2, 8, 64},
                              {"f32", 0, 4, 4, 3, 16, 32}, {"f64", 1, 16, 8, 3, 8, 32}, {"c32", 4, 2048, 8, 3, 8, 32},
                              {"c64", 5, 4096, 16, 3, 8, 64}, {"c64", 5, 4096, 16, 4, 8, 32}};
@@ -740,8 +766,8 @@ int main()
         {
             g_dtype = w.dtype;
             ProblemIn in;
-            in.A = tensor(c, c.mA, c.oA, 0);
-            in.B = tensor(c, c.mB, c.oB, 0);
+            in.A = tensor(c, c.mA, c.oA, c.padAB);
+            in.B = tensor(c, c.mB, c.oB, c.padAB);
             in.D = tensor(c, c.mD, c.oD, c.padD);
             in.bilinear = c.bilinear;
             if(c.bilinear)
@@ -767,10 +793,12 @@ int main()
                 CHECK(!avail, "%s %s: offered although byte offsets pass 2^32", w.type, c.name.c_str());
                 refused_big++;
             }
+            wide_at_4_bytes += !avail && c.padAB > 0 && v.xy_aligned == 4;
             if(!avail)
                 continue;
             const int V = 16 / w.elem_bytes;
-            CHECK(v.x_vec == V && v.y_vec == V && v.k_affine && v.K >= w.bk && (!(v.x_kfast || v.y_kfast) || v.K % V == 0) && v.xy_aligned
+            CHECK(c.padAB * w.elem_bytes % 16 == 0, "%s %s offered at %d bytes", w.type, c.name.c_str(), v.xy_aligned);
+            CHECK(v.x_vec == V && v.y_vec == V && v.k_affine && v.K >= w.bk && (!(v.x_kfast || v.y_kfast) || v.K % V == 0) && v.xy_aligned == 16
                       && (v.x_kfast || !v.shift_p) && (v.y_kfast || !v.shift_q),
                   "%s %s offered outside its restrictions", w.type, c.name.c_str());
             offered_wide++;
@@ -790,6 +818,7 @@ int main()
     CHECK(offered_mixed >= 30, "only %d mixed (case, type, tile) triples were offered a 32/64-bit direct-load kernel", offered_mixed);
     CHECK(offered_kf >= 30, "only %d k-contiguous (case, type, tile) triples were offered a 32/64-bit direct-load kernel", offered_kf);
     CHECK(offered_wide >= 60, "only %d (case, type, tile) triples were offered a 32/64-bit direct-load kernel", offered_wide);
+    CHECK(wide_at_4_bytes >= 12, "only %d (case, type, tile) triples with vectors at multiples of 4 bytes", wide_at_4_bytes);
     CHECK(refused_big >= 2, "the tensor past 2^32 bytes was not exercised (%d)", refused_big);
     std::printf("%s: %d + %d problems x tiles, %ld requests walked, %d failures\n", g_fail ? "FAILED" : "ok", offered, offered_wide, walked,
                 g_fail);
