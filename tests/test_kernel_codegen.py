@@ -22,7 +22,8 @@ _ASM = {}
 # every translation unit a test of this file looks at: the first request compiles them all, side by side
 UNITS = ["contract_f64", "contract_c32", "contract_f16_hd", "contract_f32", "contract_c64",
          "contract_f16_hk_kx", "contract_f16_hk_rx", "contract_bf16_hk_kx", "contract_bf16_hk_rx",
-         "contract_f16_hr192_kx", "contract_f16_hr192_rx", "contract_bf16_hr192_kx", "contract_bf16_hr192_rx"]
+         "contract_f16_hr192_kx", "contract_f16_hr192_rx", "contract_bf16_hr192_kx", "contract_bf16_hr192_rx",
+         "contract_f32_any", "contract_f64_any", "contract_c32_any", "contract_f16_hm", "contract_bf16_hm"]
 
 
 def device_asm(unit, tmp_path):
@@ -222,3 +223,68 @@ def test_direct_load_loops_leave_m0_alone(tmp_path):
     for a, b in main_loops(body, 128):
         text = [l for l in body[a:b] if "m0" in l.split(";")[0]]
         assert text and all(l.strip().startswith("s_add_u32 m0,") for l in text), text[:5]
+
+
+def m0_and_loads(body):
+    """In text order: "w" for a write of M0 by the load helpers, "l" for a direct load; anything else that names M0 fails."""
+    seq = []
+    for l in body:
+        code = l.split(";")[0].strip()
+        if "load_lds" in code:
+            seq.append("l")
+        elif re.search(r"\bm0\b", code):
+            assert re.match(r"s_(add_u32|mov_b32) m0,", code), code
+            seq.append("w")
+    return "".join(seq)
+
+
+@pytest.mark.parametrize("unit", ["contract_f32_any", "contract_f64_any", "contract_c32_any"])
+def test_any_element_tiles(tmp_path, unit):
+    """The 32/64-bit tiles for operands at any element: a clean ring as the others' (none of them looks for a short last tile in
+    its steps), and, over the whole kernel, one write of M0 for each load, those of the short tile included: there a lane's
+    address is selected between the two."""
+    lines = device_asm(unit, tmp_path)
+    symbols = [l.split(":")[0] for l in lines if re.match(r"^_ZN5hiptk18contract_wx_kernel.*EvNS_5KArgsE:", l)]
+    assert len(symbols) == 8, symbols
+    for symbol in symbols:
+        body = kernel_body(lines, symbol)
+        loops = main_loops(body, 16)
+        assert len(loops) == 1, f"{symbol}: {len(loops)} main loops"
+        ops = opcodes(body, *loops[0])
+        valu = sorted({o for o in ops if o.startswith("v_") and not o.startswith("v_mfma")})
+        assert not valu, f"vector ALU instructions in the main loop of {symbol}: {valu}"
+        assert not any(o.startswith(("s_cbranch", "s_branch", "buffer_store", "global_store")) for o in ops), symbol
+        assert not any("scratch_" in l for l in body), f"{symbol}: spills"
+        seq = m0_and_loads(body)
+        assert seq.count("l") >= 16 and seq == "wl" * (len(seq) // 2), (symbol, seq)
+
+
+@pytest.mark.parametrize("unit", ["contract_f16_hm", "contract_bf16_hm"])
+def test_16bit_ring_tiles_of_up_to_128_rows(tmp_path, unit):
+    """The steady loop (two K tiles): MFMAs, direct loads, LDS reads and address additions, no branch, spill or store; each of
+    its two barriers directly behind the wait for the loads of the next tile and for the wave's own LDS reads.  M0 is written by
+    the load helpers only, once for each run of loads."""
+    lines = device_asm(unit, tmp_path)
+    symbols = [l.split(":")[0] for l in lines if re.match(r"^_ZN5hiptk18contract_hm_kernel.*EvNS_5KArgsE:", l)]
+    assert len(symbols) == 12, symbols
+    for symbol in symbols:
+        bp, bq, stages = (int(x) for x in re.search(r"Li(\d+)ELi(\d+)ELi(\d+)E", symbol).groups())
+        body = kernel_body(lines, symbol)
+        a, b = main_loops(body, 16)[0]
+        ops = opcodes(body, a, b)
+        per_tile = (bp + bq) // 32  # direct loads of a wave
+        assert sum(o.startswith("v_mfma_f32_16x16x32") for o in ops) == 2 * 2 * (bp // 32) * (bq // 32), symbol
+        assert sum(o == "global_load_lds_dwordx4" for o in ops) == 2 * per_tile, symbol
+        valu = sorted({o for o in ops if o.startswith("v_") and not o.startswith("v_mfma")})
+        assert all(o.startswith(("v_add_u32", "v_lshl_add_u32", "v_lshlrev_b32")) for o in valu), f"vector ALU instructions in the main loop of {symbol}: {valu}"
+        assert not any(o.startswith(("s_cbranch", "s_branch", "buffer_store", "global_store")) for o in ops), symbol
+        assert not any("scratch_" in l for l in body), f"{symbol}: spills"
+        code = [l.split(";")[0].strip() for l in body[a:b]]
+        code = [l for l in code if l and not l.endswith(":") and not l.startswith(".")]
+        bars = [i for i, l in enumerate(code) if l.startswith("s_barrier")]
+        assert len(bars) == 2, symbol
+        for i in bars:
+            wait = code[i - 1]
+            assert wait.startswith("s_waitcnt") and f"vmcnt({(stages - 2) * per_tile})" in wait and "lgkmcnt(0)" in wait, f"{symbol}: '{wait}' in front of a barrier"
+        seq = m0_and_loads(body)
+        assert "w" in seq and seq.startswith("w") and "ww" not in seq and "lllll" not in seq, (symbol, seq)
