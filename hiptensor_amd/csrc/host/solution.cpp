@@ -323,8 +323,8 @@ namespace hipta
         else
         {
             // (the 32 x 32 tiles that take operands at any element read 64 bytes of a row per K tile and wave: off the 128-byte
-            // lines, from HBM, that comes at half the rate.  f32 15015 x 36 x 7322, both k-contiguous, 295 us on them, 134 on 64 x
-            // 64; 24 x 8746 x 5506 120 and 92.  Row-contiguous, and where operands stay in the caches, they win as their
+            // lines, from HBM, that comes at half the rate.  f32 15015 x 36 x 7322, both k-contiguous, 349 us on them, 143 on 64 x
+            // 64; 24 x 8746 x 5506 148 and 95.  Row-contiguous, and where operands stay in the caches, they win as their
             // rates say: 901 x 176 x 332 c32 11.0 and 25.1)
             us = std::max(us, bytes / (dev.hbm_gbs * 1e3 * (any_split_lines && s.bp * s.bq < 4096 ? 0.32 : 0.6)));
         }
